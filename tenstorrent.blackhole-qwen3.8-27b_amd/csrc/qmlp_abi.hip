@@ -173,19 +173,23 @@ int forward_impl(const char* fn, const void* x, const void* wg, const void* wu, 
   if (int rc = current_device_info(&di)) return rc;
   ForwardArgs a{x, (const uint8_t*)wg, (const uint8_t*)wu, (const uint8_t*)wd, residual, out, (uint8_t*)ws,
                 M, H, I, fmt, (flags & QMLP_OUT_F32) ? 1 : 0, (flags & QMLP_RESIDUAL_F32) ? 1 : 0, normw, eps};
-  // M <= 32: split-K weight streaming with LDS-staged activations (the RMSNorm fused into its
-  // staging and epilogue); where no such split fits (a K too long for the staged activations, or
-  // a device too small for the split's registers), M <= 32: stream-K
-  // weight streaming with activations read from L2; larger M: the LDS-tiled matrix-core GEMM.
-  // The last two take the RMSNorm as a separate pass.
-  if (gemv_supported(M, H, I, di.num_cus)) return launch_forward_gemv(a, di.num_cus, (hipStream_t)stream);
-  if (normw) {
+  // M <= 32: split-K weight streaming with LDS-staged activations; where no such split fits (a K
+  // too long for the staged activations, or a device too small for the split's registers),
+  // M <= 32: stream-K weight streaming with activations read from L2; larger M: the LDS-tiled
+  // matrix-core GEMM.  The RMSNorm runs as a pass of its own, or with the activation conversion
+  // where the kernels take one (block-float weights, M > 32).  Fused into the split kernel's
+  // staging, where every workgroup read every token row, it cost more than the pass and its
+  // launch: gate/up 45 against 35 us at 1 and 16 tokens, 56 against 41 us at 32 (27B, bfp8).
+  const bool gemv = gemv_supported(M, H, I, di.num_cus);
+  const bool stream_k = !gemv && stream_supported(M, H, I, di.num_cus);
+  if (normw && (gemv || stream_k || fmt == QMLP_FMT_BF16)) {
     uint8_t* xn = (uint8_t*)ws + L.xn;
     if (int rc = launch_rmsnorm(x, normw, eps, M, H, xn, (hipStream_t)stream)) return rc;
     a.x = xn;
     a.normw = nullptr;
   }
-  if (stream_supported(M, H, I, di.num_cus)) return launch_forward_stream(a, di.num_cus, (hipStream_t)stream);
+  if (gemv) return launch_forward_gemv(a, di.num_cus, (hipStream_t)stream);
+  if (stream_k) return launch_forward_stream(a, di.num_cus, (hipStream_t)stream);
   if (tiled_supported(M, H, I)) return launch_forward_tiled(a, di.num_cus, (hipStream_t)stream);
   return set_error(QMLP_E_SHAPE, "%s: no kernel for M=%d H=%d I=%d", fn, M, H, I);
 }

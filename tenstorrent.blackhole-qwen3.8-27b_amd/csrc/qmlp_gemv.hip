@@ -50,8 +50,6 @@ struct GvParams {
   int M, K, N;
   int C, T, G, S, KQ, Ng, P, maxseg;  // KQ: superblocks of the longest K split
   int x_scale;            // 1: src is bf16 and is converted to fp16 * 2^t (block-float gate/up)
-  const uint16_t* normw;  // gate/up with the RMSNorm prologue: bf16 [K] weight w (gain 1 + w)
-  float eps;              //   and its epsilon
   const int* th_in;       // block-float down: h = h16 * 2^-th[m]
   int* th_out;            // block-float gate/up: th[m] written by tile group 0
   const Trailer* tg;      // block-float gate/up: weight row-norm trailers for the h bound
@@ -100,14 +98,13 @@ struct GStage {
 // loads (vector loads complete in order: waiting for activations issued after the weights would
 // also wait for the weights).  Thread (m = token row, tl) handles chunks of 8 values at
 // K = 8 * (tl + c * TPR), c < nch = kq * MG; all MAXCH loads are unconditional (clamped chunk index).
-template <int MAXCH, bool NORM>
+template <int MAXCH>
 struct BStage {
   u32x4 v[MAXCH];
-  u32x4 w[NORM ? MAXCH : 1];  // RMSNorm weight of the same K values
 };
 
-template <int NW, int MAXCH, bool NORM, int MG>
-__device__ __forceinline__ void stage_b_issue(const GvParams& p, int k0, int kq, BStage<MAXCH, NORM>& bs) {
+template <int NW, int MAXCH, int MG>
+__device__ __forceinline__ void stage_b_issue(const GvParams& p, int k0, int kq, BStage<MAXCH>& bs) {
   constexpr int TPR = NW * 64 / (16 * MG);  // threads per token row
   const int m = threadIdx.x / TPR, tl = threadIdx.x % TPR;
   const int mr = min(m, p.M - 1);  // rows beyond M duplicate row M-1 (their outputs are discarded)
@@ -115,47 +112,11 @@ __device__ __forceinline__ void stage_b_issue(const GvParams& p, int k0, int kq,
   const uint16_t* row = p.src + (size_t)mr * p.K + k0;
 #pragma unroll
   for (int c = 0; c < MAXCH; ++c) bs.v[c] = *(const u32x4*)(row + (tl + min(c, nch - 1) * TPR) * 8);
-  if constexpr (NORM) {
-#pragma unroll
-    for (int c = 0; c < MAXCH; ++c) bs.w[c] = *(const u32x4*)(p.normw + k0 + (tl + min(c, nch - 1) * TPR) * 8);
-  }
 }
 
-// Whole-row sum of squares of token row m (RMSNorm prologue): the TPR threads of the row read it
-// in 16-byte chunks, kNormBatch loads in flight, and reduce in a fixed order, so every workgroup
-// -- whatever its K range -- computes the same value for the same row.
-constexpr int kNormBatch = 8;
-template <int TPR>
-__device__ __forceinline__ float row_sum_squares(const GvParams& p, int m, int tl) {
-  const int nfull = p.K / (TPR * 8);
-  const uint16_t* row = p.src + (size_t)min(m, p.M - 1) * p.K;
-  float sx = 0.f;
-  for (int j0 = 0; j0 < nfull; j0 += kNormBatch) {
-    u32x4 t[kNormBatch];
-#pragma unroll
-    for (int b = 0; b < kNormBatch; ++b) t[b] = *(const u32x4*)(row + (tl + min(j0 + b, nfull - 1) * TPR) * 8);
-#pragma unroll
-    for (int b = 0; b < kNormBatch; ++b)
-      if (j0 + b < nfull)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float lo = bf16_to_f32((uint16_t)(t[b][i] & 0xffffu)), hi = bf16_to_f32((uint16_t)(t[b][i] >> 16));
-          sx = fmaf(lo, lo, sx);
-          sx = fmaf(hi, hi, sx);
-        }
-  }
-#pragma unroll
-  for (int o = TPR / 2; o > 0; o >>= 1) sx += __shfl_xor(sx, o);
-  return sx;
-}
-
-// With the RMSNorm prologue the staged value is the normalised activation
-// n = bf16(x * rs * (1 + w)), rs = 1 / sqrt(mean(x^2) + eps) over the whole row -- the bf16 tensor
-// the decoder's separate norm hands to the MLP (docker/qwen-c2-graft/graft/layer.py:352-357) --
-// then converted like any activation.
-template <int NW, int MAXCH, bool NORM, int MG>
-__device__ __forceinline__ void stage_b_finish(const GvParams& p, int kq, const BStage<MAXCH, NORM>& bs,
-                                               uint8_t* ldsb, int* lds_t, float* lds_ss) {
+template <int NW, int MAXCH, int MG>
+__device__ __forceinline__ void stage_b_finish(const GvParams& p, int kq, const BStage<MAXCH>& bs, uint8_t* ldsb,
+                                               int* lds_t, float* lds_ss) {
   constexpr int TPR = NW * 64 / (16 * MG);
   const int m = threadIdx.x / TPR, tl = threadIdx.x % TPR;
   const int nch = kq * kSuperK / (TPR * 8);
@@ -163,114 +124,71 @@ __device__ __forceinline__ void stage_b_finish(const GvParams& p, int kq, const 
     const int kk = e >> 6, r = e & 63;
     return (kk * MG + (m >> 4)) * 2048 + (int)bfrag_off(r >> 4, m & 15, (r >> 3) & 1);
   };
-  if (!p.x_scale && !NORM) {
+  if (!p.x_scale) {
 #pragma unroll
     for (int c = 0; c < MAXCH; ++c)
       if (c < nch) *(u32x4*)(ldsb + lds_off((tl + c * TPR) * 8)) = bs.v[c];
     return;
   }
-  if constexpr (!NORM) {
-    // bf16 x -> fp16 * 2^t on packed 16-bit words: the magnitudes' integer maximum is the
-    // maximum value, the sum of squares comes from v_dot2_f32_bf16, and the conversion is
-    // fp16 bits = ((|x| bits - ((112 - t) << 7)) << 3) | sign, exact while x * 2^t is a normal
-    // half; values below 2^-14 after scaling (2^-28 of the range maximum) are flushed to zero.
-    u16x2 mx2 = {0, 0};
-    float ss = 0.f;
+  // bf16 x -> fp16 * 2^t on packed 16-bit words: the magnitudes' integer maximum is the
+  // maximum value, the sum of squares comes from v_dot2_f32_bf16, and the conversion is
+  // fp16 bits = ((|x| bits - ((112 - t) << 7)) << 3) | sign, exact while x * 2^t is a normal
+  // half; values below 2^-14 after scaling (2^-28 of the range maximum) are flushed to zero.
+  u16x2 mx2 = {0, 0};
+  float ss = 0.f;
 #pragma unroll
-    for (int c = 0; c < MAXCH; ++c)
-      if (c < nch)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint32_t r = bs.v[c][i];
-          mx2 = __builtin_elementwise_max(mx2, __builtin_bit_cast(u16x2, r & 0x7fff7fffu));
-          ss = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, r), __builtin_bit_cast(bf16x2, r), ss, false);
-        }
-    uint32_t mb = max((uint32_t)mx2.x, (uint32_t)mx2.y);
-#pragma unroll
-    for (int o = TPR / 2; o > 0; o >>= 1) {
-      mb = max(mb, (uint32_t)__shfl_xor((int)mb, o));
-      ss += __shfl_xor(ss, o);
-    }
-    const float mxf = bf16_to_f32((uint16_t)mb);
-    int e2 = 0;
-    if (mxf > 0.f) frexpf(mxf, &e2);
-    const int t = mxf > 0.f ? min(15 - e2, 112) : 0;
-    if (tl == 0) {
-      lds_t[m] = t;
-      lds_ss[m] = ss;
-    }
-    const uint32_t dd = (uint32_t)(112 - t) << 7;
-    const u16x2 d2 = __builtin_bit_cast(u16x2, dd | (dd << 16));
-#pragma unroll
-    for (int c = 0; c < MAXCH; ++c) {
-      if (c < nch) {
-        uint32_t o[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint32_t r = bs.v[c][i];
-          const u16x2 sub = __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, r & 0x7fff7fffu), d2);
-          o[i] = __builtin_bit_cast(uint32_t, (u16x2)(sub << (u16x2){3, 3})) | (r & 0x80008000u);
-        }
-        *(u32x4*)(ldsb + lds_off((tl + c * TPR) * 8)) = u32x4{o[0], o[1], o[2], o[3]};
-      }
-    }
-    return;
-  }
-  float rs = 1.0f;
-  if constexpr (NORM) rs = 1.0f / sqrtf(row_sum_squares<TPR>(p, m, tl) / (float)p.K + p.eps);
-  auto value = [&](int c, int i, int hi) {
-    const float xr = bf16_to_f32((uint16_t)(hi ? bs.v[c][i] >> 16 : bs.v[c][i] & 0xffffu));
-    if constexpr (NORM) {
-      const float wv = bf16_to_f32((uint16_t)(hi ? bs.w[c][i] >> 16 : bs.w[c][i] & 0xffffu));
-      return bf16_to_f32(f32_to_bf16(xr * rs * (1.0f + wv)));
-    }
-    return xr;
-  };
-  // block float: value -> fp16 * 2^t with max|value| * 2^t in [2^14, 2^15) over this K range
-  // (exact unless a value is 2^31 times smaller than the range maximum).  The range's sum of
-  // squares feeds the h bound.
-  float mx = 0.f, ss = 0.f;
-#pragma unroll
-  for (int c = 0; c < MAXCH; ++c) {
-    if (c < nch) {
+  for (int c = 0; c < MAXCH; ++c)
+    if (c < nch)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-#pragma unroll
-        for (int hi = 0; hi < 2; ++hi) {
-          const float v = value(c, i, hi);
-          mx = fmaxf(mx, fabsf(v));
-          ss = fmaf(v, v, ss);
-        }
+        const uint32_t r = bs.v[c][i];
+        mx2 = __builtin_elementwise_max(mx2, __builtin_bit_cast(u16x2, r & 0x7fff7fffu));
+        ss = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, r), __builtin_bit_cast(bf16x2, r), ss, false);
       }
-    }
-  }
-  // reduce over the TPR threads of this row (a fixed tree inside one wave: deterministic)
+  uint32_t mb = max((uint32_t)mx2.x, (uint32_t)mx2.y);
 #pragma unroll
   for (int o = TPR / 2; o > 0; o >>= 1) {
-    mx = fmaxf(mx, __shfl_xor(mx, o));
+    mb = max(mb, (uint32_t)__shfl_xor((int)mb, o));
     ss += __shfl_xor(ss, o);
   }
+  const float mxf = bf16_to_f32((uint16_t)mb);
   int e2 = 0;
-  if (mx > 0.f) frexpf(mx, &e2);
-  const int t = (p.x_scale && mx > 0.f) ? 15 - e2 : 0;
+  if (mxf > 0.f) frexpf(mxf, &e2);
+  const int t = mxf > 0.f ? min(15 - e2, 112) : 0;
   if (tl == 0) {
     lds_t[m] = t;
     lds_ss[m] = ss;
   }
+  const uint32_t dd = (uint32_t)(112 - t) << 7;
+  const u16x2 d2 = __builtin_bit_cast(u16x2, dd | (dd << 16));
 #pragma unroll
   for (int c = 0; c < MAXCH; ++c) {
     if (c < nch) {
       uint32_t o[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float a = value(c, i, 0), b = value(c, i, 1);
-        if (p.x_scale)
-          o[i] = (uint32_t)f32_to_f16_bits(__builtin_amdgcn_ldexpf(a, t)) |
-                 ((uint32_t)f32_to_f16_bits(__builtin_amdgcn_ldexpf(b, t)) << 16);
-        else
-          o[i] = (uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16);
+        const uint32_t r = bs.v[c][i];
+        const u16x2 sub = __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, r & 0x7fff7fffu), d2);
+        o[i] = __builtin_bit_cast(uint32_t, (u16x2)(sub << (u16x2){3, 3})) | (r & 0x80008000u);
       }
       *(u32x4*)(ldsb + lds_off((tl + c * TPR) * 8)) = u32x4{o[0], o[1], o[2], o[3]};
+    }
+  }
+  // The word arithmetic above has no infinities or NaN: a row slice that holds one is staged again
+  // with them (rare, decided once per row).
+  if (mb >= 0x7f80u) {
+    auto half = [](uint32_t b) {  // finite values: any, the row's products are not finite anyway
+      const uint32_t m = b & 0x7fffu;
+      return m < 0x7f80u ? 0x3c00u : (m == 0x7f80u ? 0x7c00u | (b & 0x8000u) : 0x7e00u);
+    };
+#pragma unroll
+    for (int c = 0; c < MAXCH; ++c) {
+      if (c < nch) {
+        uint32_t o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = half(bs.v[c][i] & 0xffffu) | (half(bs.v[c][i] >> 16) << 16);
+        *(u32x4*)(ldsb + lds_off((tl + c * TPR) * 8)) = u32x4{o[0], o[1], o[2], o[3]};
+      }
     }
   }
 }
@@ -454,7 +372,7 @@ __device__ __forceinline__ void gepilogue(const GvParams& p, int t, const f32x4 
 
 // ---------------------------------------------------------------- kernel
 
-template <int WF, int NMAT, int NW, int MAXCH, bool NORM, int MG>
+template <int WF, int NMAT, int NW, int MAXCH, int MG>
 __global__ __launch_bounds__(NW * 64) void gemv_kernel(GvParams p) {
   constexpr int SPS = WF ? 4 : 2;  // K-steps per register stage
   constexpr int SPU = kSteps / SPS;
@@ -502,11 +420,11 @@ __global__ __launch_bounds__(NW * 64) void gemv_kernel(GvParams p) {
   if (nst > 1) gadvance<SPU>(P1, kq);
   P2 = P1;
   if (nst > 2) gadvance<SPU>(P2, kq);
-  BStage<MAXCH, NORM> bs;
-  stage_b_issue<NW, MAXCH, NORM, MG>(p, c0 * kSuperK, kq, bs);
+  BStage<MAXCH> bs;
+  stage_b_issue<NW, MAXCH, MG>(p, c0 * kSuperK, kq, bs);
   gload(s0, p, blk_base, P0, lw, le);
   gload(s1, p, blk_base, P1, lw, le);  // repeats stage 0 when nst == 1
-  stage_b_finish<NW, MAXCH, NORM, MG>(p, kq, bs, ldsb, s_t, s_ss);
+  stage_b_finish<NW, MAXCH, MG>(p, kq, bs, ldsb, s_t, s_ss);
   gload(s2, p, blk_base, P2, lw, le);
   __syncthreads();
 
@@ -868,9 +786,9 @@ static int enable_large_lds(const void* kern, const char* what) {
   return 0;
 }
 
-template <int WF, int NMAT, int MAXCH, bool NORM, int MG>
+template <int WF, int NMAT, int MAXCH, int MG>
 static int launch_gemv_ch(const GvParams& p, size_t lds, hipStream_t s) {
-  auto kern = gemv_kernel<WF, NMAT, kGemvNW, MAXCH, NORM, MG>;
+  auto kern = gemv_kernel<WF, NMAT, kGemvNW, MAXCH, MG>;
   if (int rc = enable_large_lds((const void*)kern, "gemv_kernel")) return rc;
   launch_timed(NMAT == 2 ? 0 : 1, kern, dim3(p.P), dim3(kGemvNW * 64), lds, s, p);
   return check_launch("gemv_kernel");
@@ -878,17 +796,17 @@ static int launch_gemv_ch(const GvParams& p, size_t lds, hipStream_t s) {
 
 // The staging register array is sized by a small set of buckets (loads beyond KQ * MG are clamped
 // duplicates).
-template <int WF, int NMAT, bool NORM, int MG>
+template <int WF, int NMAT, int MG>
 static int launch_gemv_mg(const GvParams& p, size_t lds, hipStream_t s) {
   const int nch = p.KQ * MG;
-  if (nch <= 4) return launch_gemv_ch<WF, NMAT, 4, NORM, MG>(p, lds, s);
-  if (nch <= 10) return launch_gemv_ch<WF, NMAT, 10, NORM, MG>(p, lds, s);
-  return launch_gemv_ch<WF, NMAT, kGemvMaxChunks, NORM, MG>(p, lds, s);
+  if (nch <= 4) return launch_gemv_ch<WF, NMAT, 4, MG>(p, lds, s);
+  if (nch <= 10) return launch_gemv_ch<WF, NMAT, 10, MG>(p, lds, s);
+  return launch_gemv_ch<WF, NMAT, kGemvMaxChunks, MG>(p, lds, s);
 }
 
-template <int WF, int NMAT, bool NORM = false>
+template <int WF, int NMAT>
 static int launch_gemv(const GvParams& p, int mg, size_t lds, hipStream_t s) {
-  return mg == 2 ? launch_gemv_mg<WF, NMAT, NORM, 2>(p, lds, s) : launch_gemv_mg<WF, NMAT, NORM, 1>(p, lds, s);
+  return mg == 2 ? launch_gemv_mg<WF, NMAT, 2>(p, lds, s) : launch_gemv_mg<WF, NMAT, 1>(p, lds, s);
 }
 
 size_t gemv_part_bytes(int rows, int K, int nmat, int mg) {
@@ -943,8 +861,6 @@ int launch_forward_gemv(const ForwardArgs& a, int num_cus, hipStream_t s) {
   g.P = pg.P;
   g.maxseg = pg.maxseg;
   g.x_scale = fmt != 0;
-  g.normw = (const uint16_t*)a.normw;
-  g.eps = a.eps;
   g.th_out = th;
   g.tg = (const Trailer*)(a.wg + trailer_offset(a.I, a.H, fmt));
   g.tu = (const Trailer*)(a.wu + trailer_offset(a.I, a.H, fmt));
@@ -953,13 +869,9 @@ int launch_forward_gemv(const ForwardArgs& a, int num_cus, hipStream_t s) {
   g.pss = (float*)(a.ws + L.pss);
   g.counters = (int*)(a.ws + L.counters_gu);
   const size_t lg = gemv_lds_bytes(pg, 2, mg);
-  int rc;
-  if (fmt == 2)
-    rc = a.normw ? launch_gemv<2, 2, true>(g, mg, lg, s) : launch_gemv<2, 2>(g, mg, lg, s);
-  else if (fmt == 1)
-    rc = a.normw ? launch_gemv<1, 2, true>(g, mg, lg, s) : launch_gemv<1, 2>(g, mg, lg, s);
-  else
-    rc = a.normw ? launch_gemv<0, 2, true>(g, mg, lg, s) : launch_gemv<0, 2>(g, mg, lg, s);
+  int rc = fmt == 2   ? launch_gemv<2, 2>(g, mg, lg, s)
+           : fmt == 1 ? launch_gemv<1, 2>(g, mg, lg, s)
+                      : launch_gemv<0, 2>(g, mg, lg, s);
   if (rc) return rc;
   GvParams d{};
   d.w0 = a.wd;
