@@ -94,6 +94,15 @@ int qmlp_pack(const void* src0, const void* src1, int rows, int cols, int fmt, v
 int qmlp_packed_info(const void* packed, int rows, int cols, int fmt, double* max_row_norm,
                      uint32_t* flushed_groups, qmlp_stream_t stream);
 
+/* qmlp_quantize_bfp8 / _bf4 and qmlp_pack in one pass: bf16 [rows,cols] -> the same packed bytes in
+ * any format, without the canonical intermediates.  qmlp_quantize_pack_info reads the trailer back
+ * like qmlp_packed_info and also the number of groups that hold a non-finite value (packed as
+ * zeros; a matrix with such groups must not be used; always 0 for QMLP_FMT_BF16). */
+int qmlp_quantize_pack(const void* w_bf16, int rows, int cols, int fmt, void* packed,
+                       size_t packed_bytes, qmlp_stream_t stream);
+int qmlp_quantize_pack_info(const void* packed, int rows, int cols, int fmt, double* max_row_norm,
+                            uint32_t* flushed_groups, uint32_t* bad_groups, qmlp_stream_t stream);
+
 /* Inverse of qmlp_pack for bfp8 (lossless for every group that was not flushed): packed ->
  * canonical q/e8.  Used by the on-disk weight cache and the packing audit (the reference audits
  * its packed gate/up the same way, packed_weight_check.cpp:1-37). */

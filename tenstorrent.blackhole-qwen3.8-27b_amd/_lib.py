@@ -34,6 +34,9 @@ SIGNATURES = {
     "qmlp_packed_bytes": (_SZ, [_I, _I, _I]),
     "qmlp_pack": (_I, [_P, _P, _I, _I, _I, _P, _SZ, _P]),
     "qmlp_packed_info": (_I, [_P, _I, _I, _I, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_uint32), _P]),
+    "qmlp_quantize_pack": (_I, [_P, _I, _I, _I, _P, _SZ, _P]),
+    "qmlp_quantize_pack_info": (_I, [_P, _I, _I, _I, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_uint32),
+                                     ctypes.POINTER(ctypes.c_uint32), _P]),
     "qmlp_unpack_bfp8": (_I, [_P, _I, _I, _P, _P, _P]),
     "qmlp_unpack_bf4": (_I, [_P, _I, _I, _P, _P, _P]),
     "qmlp_dequant_packed": (_I, [_P, _I, _I, _I, _P, _P]),

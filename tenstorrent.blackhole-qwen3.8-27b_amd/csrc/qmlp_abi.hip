@@ -249,23 +249,51 @@ int qmlp_pack(const void* src0, const void* src1, int rows, int cols, int fmt, v
   return launch_pack(src0, src1, rows, cols, fmt, packed, (hipStream_t)stream);
 }
 
-int qmlp_packed_info(const void* packed, int rows, int cols, int fmt, double* max_row_norm, uint32_t* flushed_groups,
-                     qmlp_stream_t stream) {
-  if (!packed) return set_error(QMLP_E_NULL, "qmlp_packed_info: null pointer");
-  if (!shape_ok(rows, cols) || !known_fmt(fmt)) return set_error(QMLP_E_SHAPE, "qmlp_packed_info: bad shape/format");
+int qmlp_quantize_pack(const void* w_bf16, int rows, int cols, int fmt, void* packed, size_t packed_bytes,
+                       qmlp_stream_t stream) {
+  const char* fn = "qmlp_quantize_pack";
+  if (!known_fmt(fmt)) return set_error(QMLP_E_FORMAT, "%s: unknown format %d", fn, fmt);
+  if (!w_bf16 || !packed) return set_error(QMLP_E_NULL, "%s: null pointer", fn);
+  if (!shape_ok(rows, cols))
+    return set_error(QMLP_E_SHAPE, "%s: rows must be a multiple of 16 and cols of 256 (%dx%d)", fn, rows, cols);
+  if (!aligned16(w_bf16) || !aligned16(packed)) return set_error(QMLP_E_ALIGN, "%s: misaligned pointer", fn);
+  if (packed_bytes < packed_total(rows, cols, fmt))
+    return set_error(QMLP_E_WORKSPACE, "%s: packed buffer holds %zu bytes, needs %zu", fn, packed_bytes,
+                     packed_total(rows, cols, fmt));
   DeviceInfo di;
   if (int rc = current_device_info(&di)) return rc;
-  Trailer t;
+  return launch_quantize_pack(w_bf16, rows, cols, fmt, packed, (hipStream_t)stream);
+}
+
+static int info_impl(const char* fn, const void* packed, int rows, int cols, int fmt, double* max_row_norm,
+                     uint32_t* flushed_groups, uint32_t* bad_groups, qmlp_stream_t stream) {
+  if (!packed) return set_error(QMLP_E_NULL, "%s: null pointer", fn);
+  if (!shape_ok(rows, cols) || !known_fmt(fmt)) return set_error(QMLP_E_SHAPE, "%s: bad shape/format", fn);
+  DeviceInfo di;
+  if (int rc = current_device_info(&di)) return rc;
+  PackTrailer t;
   const uint8_t* src = (const uint8_t*)packed + trailer_offset(rows, cols, fmt);
   if (hipMemcpyAsync(&t, src, sizeof(t), hipMemcpyDeviceToHost, (hipStream_t)stream) != hipSuccess ||
       hipStreamSynchronize((hipStream_t)stream) != hipSuccess)
-    return set_error(QMLP_E_LAUNCH, "qmlp_packed_info: copy failed");
-  if (t.magic != kTrailerMagic) return set_error(QMLP_E_FORMAT, "qmlp_packed_info: buffer was not packed by qmlp_pack");
+    return set_error(QMLP_E_LAUNCH, "%s: copy failed", fn);
+  if (t.magic != kTrailerMagic) return set_error(QMLP_E_FORMAT, "%s: buffer was not packed by qmlp_pack", fn);
   double n;
   memcpy(&n, &t.max_row_norm_bits, sizeof(n));
   if (max_row_norm) *max_row_norm = n;
   if (flushed_groups) *flushed_groups = t.flushed_groups;
+  if (bad_groups) *bad_groups = t.bad_groups;
   return 0;
+}
+
+int qmlp_packed_info(const void* packed, int rows, int cols, int fmt, double* max_row_norm, uint32_t* flushed_groups,
+                     qmlp_stream_t stream) {
+  return info_impl("qmlp_packed_info", packed, rows, cols, fmt, max_row_norm, flushed_groups, nullptr, stream);
+}
+
+int qmlp_quantize_pack_info(const void* packed, int rows, int cols, int fmt, double* max_row_norm,
+                            uint32_t* flushed_groups, uint32_t* bad_groups, qmlp_stream_t stream) {
+  return info_impl("qmlp_quantize_pack_info", packed, rows, cols, fmt, max_row_norm, flushed_groups, bad_groups,
+                   stream);
 }
 
 static int unpack_impl(const char* fn, const void* packed, int rows, int cols, int fmt, void* q, void* e8,

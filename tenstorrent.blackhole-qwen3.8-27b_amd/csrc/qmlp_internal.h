@@ -5,7 +5,15 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "qmlp_common.h"
+
 namespace qmlp {
+
+// The trailer as qmlp_quantize_pack writes it: the padding word after the magic counts the groups
+// with non-finite values (0 in a valid matrix).
+struct PackTrailer : Trailer {
+  uint32_t bad_groups;
+};
 
 // Error reporting (thread-local message, set by the C ABI layer and the launchers).
 int set_error(int code, const char* fmt, ...);
@@ -40,6 +48,7 @@ void launch_timed(int slot, void (*kern)(Args...), dim3 grid, dim3 block, size_t
 // Load-time kernels (qmlp_pack.hip).
 int launch_quantize(const void* w, int rows, int cols, void* q, void* e8, uint32_t* bad, int mbits, hipStream_t s);
 int launch_pack(const void* src0, const void* src1, int rows, int cols, int fmt, void* packed, hipStream_t s);
+int launch_quantize_pack(const void* w, int rows, int cols, int fmt, void* packed, hipStream_t s);
 int launch_unpack(const void* packed, int rows, int cols, int fmt, void* q, void* e8, hipStream_t s);
 int launch_dequant(const void* packed, int rows, int cols, int fmt, float* out, hipStream_t s);
 int launch_fill_zero(void* p, size_t bytes, hipStream_t s);

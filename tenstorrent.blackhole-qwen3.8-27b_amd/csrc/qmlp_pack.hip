@@ -377,6 +377,247 @@ __global__ void dequant_bf16_kernel(const uint8_t* __restrict__ packed, int rows
   }
 }
 
+// ---------------------------------------------------------------- quantise and pack in one pass
+//
+// bf16 weights -> packed layout, the same bytes as quantize_kernel / rowinfo / pack kernels leave,
+// with one read of the weights and one write of the packed matrix.  Those passes write and re-read
+// the canonical mantissas and exponents.  us per 27B matrix, 17408 x 5120 and 5120 x 17408: bfp8
+// 77 + 205 + 34 and 77 + 68 + 34 there, 62 and 74 here (4.4 and 3.7 TB/s); bf4 80 + 202 + 26, here
+// 56; bf16 weights 215 + 60 and 130 + 60, here 89 and 83.
+//
+// Bound by memory.  One block of 8 waves per 16-row tile; lane l = 16 quarter + row holds one
+// 16-value group, the unit of the packed layout, so a wave's step reads 128 contiguous bytes of 16
+// rows and writes 1 KB.  The mantissas do not depend on the row's base exponent and leave at once;
+// the shared exponents wait (in LDS, or in their own place in the packed matrix for rows too long
+// for it) until the row's largest is known.  The next superblock is in flight while one is
+// converted (64 KB per block).  The 5120-row matrix has 320 blocks for 256 CUs, hence its lower rate.
+//
+// Row norms are sums in double precision in rowinfo's order -- accumulator t of 256 takes the
+// groups t, t + 256, ..., then halves are added, t + 128 first -- so that they are the same bits:
+// wave w takes superblocks w, w + 8, ..., whose groups belong to accumulators 16 (sb % 16) + 4 j +
+// quarter, i.e. 2 x 4 per lane.
+
+constexpr int kPackWaves = 8;
+constexpr int kPackLdsExp = 176;  // superblocks whose exponent words fit beside the norm sums in 64 KB of LDS
+
+struct PackedGroup {
+  uint32_t d[4];  // bfp8: 16 bytes excess-128; bf4: two dwords of nibbles excess-8
+  uint32_t e;     // shared exponent, 0: all zero or not finite
+  int sq;         // sum of the squared mantissas
+  bool finite;
+};
+
+// One group: q = round-half-even(v * 2^(127 - e)) clamped to 2^MB - 1 magnitudes, e from the largest
+// magnitude.  v has 8 significant bits and the scale is a power of two, so the product is exact
+// (or far below 1/2); adding 1.5 * 2^23 rounds it half to even into the low mantissa bits.
+template <int MB>
+__device__ __forceinline__ PackedGroup quantize_group(u32x4 lo, u32x4 hi) {
+  PackedGroup o;
+  uint32_t mx = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    mx = max(mx, max(lo[i] & 0x7fffu, (lo[i] >> 16) & 0x7fffu));
+    mx = max(mx, max(hi[i] & 0x7fffu, (hi[i] >> 16) & 0x7fffu));
+  }
+  o.finite = mx < 0x7f80u;
+  const bool live = o.finite && mx != 0;
+  const int e = max(1, (int)(mx >> 7) + 1 - MB);
+  o.e = live ? (uint32_t)e : 0u;
+  constexpr float TOP = (float)((1 << MB) - 1);
+  constexpr float BIAS = 12582912.0f + (float)(1 << MB);  // 1.5 * 2^23: round, and the excess
+  uint32_t u[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const uint32_t w = i < 8 ? lo[i / 2] : hi[i / 2 - 4];
+    const float v = __uint_as_float((i & 1) ? (w & 0xffff0000u) : (w << 16));
+    const float x = fminf(fmaxf(__builtin_amdgcn_ldexpf(v, 127 - e), -TOP), TOP);
+    u[i] = live ? __float_as_uint(x + BIAS) & 0xffu : (uint32_t)(1 << MB);
+  }
+  uint32_t b[4];  // bytes in value order
+#pragma unroll
+  for (int i = 0; i < 4; ++i) b[i] = u[4 * i] | (u[4 * i + 1] << 8) | (u[4 * i + 2] << 16) | (u[4 * i + 3] << 24);
+  int sq = MB == 7 ? 0 : 16 * 64;  // bf4: sum (u - 8)^2 = sum u^2 - 16 sum u + 16 * 64
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (MB == 7) {
+      const int m = (int)(b[i] ^ 0x80808080u);
+      sq = __builtin_amdgcn_sdot4(m, m, sq, false);
+    } else {
+      sq = __builtin_amdgcn_sdot4((int)b[i], (int)b[i], sq, false);
+      sq = __builtin_amdgcn_sdot4((int)b[i], (int)0xf0f0f0f0u, sq, false);  // -16 in every byte
+    }
+  }
+  o.sq = sq;
+  if constexpr (MB == 7) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o.d[i] = b[i];
+  } else {  // byte b of dword h: u[8 h + b] | u[8 h + b + 4] << 4
+    o.d[0] = b[0] | (b[1] << 4);
+    o.d[1] = b[2] | (b[3] << 4);
+    o.d[2] = o.d[3] = 0;
+  }
+  return o;
+}
+
+// The block's row norms from acc[wave][j][lane] (accumulators t and t + 128 already added), by wave
+// 0: row lane % 16, the result in lanes 0..15; then the trailer's maximum.
+__device__ __forceinline__ void finish_norms(double sum, int lane, Trailer* tr) {
+  unsigned long long n = (unsigned long long)__double_as_longlong(sqrt(sum));
+  if (lane >= 16) n = 0;
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) {
+    const unsigned long long other = __shfl_xor(n, o);
+    n = n > other ? n : other;
+  }
+  if (lane == 0) atomicMax(&tr->max_row_norm_bits, n);
+}
+
+template <int MB, bool EXP_LDS>
+__global__ __launch_bounds__(kPackWaves * 64, 4) void quantize_pack_kernel(const uint16_t* __restrict__ w, int cols,
+                                                                       uint8_t* __restrict__ packed,
+                                                                       int* __restrict__ rowexp, PackTrailer* tr) {
+  constexpr int BLK = MB == 7 ? kBfp8Block : kBf4Block;
+  extern __shared__ uint32_t s_e[];  // EXP_LDS: [C][64] shared exponents, byte j of a lane's word: K-step j
+  __shared__ double s_acc[kPackWaves][kSteps][64];
+  __shared__ int s_max[kPackWaves][16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, C = cols / kSuperK;
+  const int row = blockIdx.x * kTileRows + (lane & 15);
+  const uint16_t* src = w + (size_t)row * cols + (lane >> 4) * 16;
+  uint8_t* dst = packed + (size_t)blockIdx.x * C * BLK;
+  u32x4 v[kSteps][2];
+  auto load = [&](int j, int sb) {
+    const uint16_t* s = src + (size_t)min(sb, C - 1) * kSuperK + j * 64;
+    v[j][0] = *(const u32x4*)s;
+    v[j][1] = *(const u32x4*)(s + 8);
+  };
+  auto exponents = [&](int sb) {
+    return EXP_LDS ? s_e + sb * 64 + lane : (uint32_t*)(dst + (size_t)sb * BLK + (BLK - 256) + lane * 4);
+  };
+  double acc[2][kSteps] = {};
+  int emax = 0;
+  uint32_t bad = 0;
+  // converts superblock sb and requests the wave's next one, K-step by K-step
+  auto convert = [&](int sb, double(&a)[kSteps]) {
+    uint8_t* blk = dst + (size_t)sb * BLK;
+    uint32_t ew = 0;
+    u32x4 pair;  // bf4: two K-steps share a 16-byte slot
+#pragma unroll
+    for (int j = 0; j < kSteps; ++j) {
+      const PackedGroup g = quantize_group<MB>(v[j][0], v[j][1]);
+      load(j, sb + kPackWaves);
+      if constexpr (MB == 7) {
+        *(u32x4*)(blk + j * 1024 + lane * 16) = u32x4{g.d[0], g.d[1], g.d[2], g.d[3]};
+      } else {
+        pair[2 * (j & 1)] = g.d[0];
+        pair[2 * (j & 1) + 1] = g.d[1];
+        if (j & 1) *(u32x4*)(blk + (j >> 1) * 1024 + lane * 16) = pair;
+      }
+      ew |= g.e << (8 * j);
+      emax = max(emax, (int)g.e);
+      bad += g.finite ? 0u : 1u;
+      a[j] += ldexp((double)g.sq, 2 * ((int)g.e - 127));
+    }
+    *exponents(sb) = ew;
+  };
+#pragma unroll
+  for (int j = 0; j < kSteps; ++j) load(j, wave);
+  for (int sb = wave; sb < C; sb += 2 * kPackWaves) {
+    convert(sb, acc[0]);
+    if (sb + kPackWaves < C) convert(sb + kPackWaves, acc[1]);
+  }
+  emax = max(emax, __shfl_xor(emax, 16));
+  emax = max(emax, __shfl_xor(emax, 32));
+  if (lane < 16) s_max[wave][lane] = emax;
+#pragma unroll
+  for (int j = 0; j < kSteps; ++j) s_acc[wave][j][lane] = acc[0][j] + acc[1][j];
+  if (bad) atomicAdd(&tr->bad_groups, bad);
+  __syncthreads();
+  int base = 0;
+#pragma unroll
+  for (int v = 0; v < kPackWaves; ++v) base = max(base, s_max[v][lane & 15]);
+  uint32_t flushed = 0;
+  for (int sb = wave; sb < C; sb += kPackWaves) {
+    const uint32_t ew = *exponents(sb);  // this thread's own words
+    uint32_t o = 0;
+#pragma unroll
+    for (int j = 0; j < kSteps; ++j) {
+      const int e = (int)((ew >> (8 * j)) & 0xffu), e5 = e - base + 20;
+      if (e && e5 < 1) ++flushed;
+      o |= ((e && e5 >= 1) ? (uint32_t)(e5 << 2) : 0u) << (8 * j);
+    }
+    *(uint32_t*)(dst + (size_t)sb * BLK + (BLK - 256) + lane * 4) = o;
+  }
+  if (flushed) atomicAdd(&tr->flushed_groups, flushed);
+  if (wave == 0) {
+    double s[kSteps];
+#pragma unroll
+    for (int j = 0; j < kSteps; ++j) {  // accumulator bits 6, 5, 4: waves v + 4, v + 2, v + 1
+      double t[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) t[v] = s_acc[v][j][lane] + s_acc[v + 4][j][lane];
+      s[j] = (t[0] + t[2]) + (t[1] + t[3]);
+    }
+    double sum = (s[0] + s[2]) + (s[1] + s[3]);  // bits 3, 2: K-steps
+    sum += __shfl_xor(sum, 32);                  // bits 1, 0: quarters
+    sum += __shfl_xor(sum, 16);
+    if (lane < 16) rowexp[row] = base - 132;
+    finish_norms(sum, lane, tr);
+  }
+}
+
+// bf16 weights: the packed layout is a permutation; wave (j, h) moves its 8 values per lane of every
+// superblock in order, which are accumulators t = 64 j + 16 quarter + 8 h + 0..7 of the row norm.
+__global__ __launch_bounds__(kPackWaves * 64) void pack_bf16_fused_kernel(const uint16_t* __restrict__ w, int cols,
+                                                                         uint8_t* __restrict__ packed,
+                                                                         int* __restrict__ rowexp, Trailer* tr) {
+  constexpr int DEPTH = 4;  // superblocks in flight per wave
+  __shared__ double s_acc[kPackWaves][8][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, C = cols / kSuperK;
+  const int j = wave >> 1, h = wave & 1;
+  const int row = blockIdx.x * kTileRows + (lane & 15);
+  const uint16_t* src = w + (size_t)row * cols + j * 64 + (lane >> 4) * 16 + h * 8;
+  uint8_t* dst = packed + (size_t)blockIdx.x * C * kBf16Block + j * 2048 + h * 1024 + lane * 16;
+  double acc[8] = {};
+  u32x4 v[DEPTH];
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) v[d] = *(const u32x4*)(src + (size_t)min(d, C - 1) * kSuperK);
+  for (int s0 = 0; s0 < C; s0 += DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      const int sb = s0 + d;
+      if (sb < C) {
+        const u32x4 t = v[d];
+        v[d] = *(const u32x4*)(src + (size_t)min(sb + DEPTH, C - 1) * kSuperK);
+        *(u32x4*)(dst + (size_t)sb * kBf16Block) = t;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const double x = (double)__uint_as_float((i & 1) ? (t[i / 2] & 0xffff0000u) : (t[i / 2] << 16));
+          acc[i] += x * x;
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) s_acc[wave][i][lane] = acc[i];
+  __syncthreads();
+  if (wave != 0) return;
+  double s[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    double t[2];
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh) {  // bits 7, 6: K-steps; bits 5, 4: quarters
+      t[hh] = (s_acc[hh][i][lane] + s_acc[4 + hh][i][lane]) + (s_acc[2 + hh][i][lane] + s_acc[6 + hh][i][lane]);
+      t[hh] += __shfl_xor(t[hh], 32);
+      t[hh] += __shfl_xor(t[hh], 16);
+    }
+    s[i] = t[0] + t[1];  // bit 3: half
+  }
+  const double sum = ((s[0] + s[4]) + (s[2] + s[6])) + ((s[1] + s[5]) + (s[3] + s[7]));
+  if (lane < 16) rowexp[row] = 0;
+  finish_norms(sum, lane, tr);
+}
+
 __global__ void fill_zero_kernel(u32x4* __restrict__ p, size_t n16) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += (size_t)gridDim.x * blockDim.x)
     p[i] = u32x4{0u, 0u, 0u, 0u};
@@ -422,6 +663,25 @@ int launch_pack(const void* src0, const void* src1, int rows, int cols, int fmt,
                        cols, base);
   }
   return check_launch("pack kernels");
+}
+
+int launch_quantize_pack(const void* w, int rows, int cols, int fmt, void* packed, hipStream_t s) {
+  uint8_t* base = (uint8_t*)packed;
+  int* rowexp = (int*)(base + rowexp_offset(rows, cols, fmt));
+  PackTrailer* tr = (PackTrailer*)(base + trailer_offset(rows, cols, fmt));
+  const dim3 grid(rows / kTileRows), block(kPackWaves * 64);
+  hipLaunchKernelGGL(trailer_init_kernel, dim3(1), dim3(64), 0, s, (Trailer*)tr);
+  if (fmt == 0) {
+    hipLaunchKernelGGL(pack_bf16_fused_kernel, grid, block, 0, s, (const uint16_t*)w, cols, base, rowexp,
+                       (Trailer*)tr);
+  } else {
+    const int C = cols / kSuperK;
+    const bool in_lds = C <= kPackLdsExp;
+    auto kern = fmt == 1 ? (in_lds ? quantize_pack_kernel<7, true> : quantize_pack_kernel<7, false>)
+                         : (in_lds ? quantize_pack_kernel<3, true> : quantize_pack_kernel<3, false>);
+    hipLaunchKernelGGL(kern, grid, block, in_lds ? (size_t)C * 256 : 0, s, (const uint16_t*)w, cols, base, rowexp, tr);
+  }
+  return check_launch("quantize_pack_kernel");
 }
 
 int launch_unpack(const void* packed, int rows, int cols, int fmt, void* q, void* e8, hipStream_t s) {

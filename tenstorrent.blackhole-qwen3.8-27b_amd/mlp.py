@@ -139,25 +139,44 @@ def pack_canonical(q, e8, fmt="bfp8", strict=True, stream=None):
     return pw
 
 
-def pack_weight(w, fmt="bfp8", strict=True, stream=None):
-    """bf16 ``[rows, cols]`` GPU tensor (HF layout: [out, in]) -> PackedWeight in the matrix format
-    ``fmt`` ("bf16", "bfp8" or "bf4")."""
+def _pack_weight_begin(w, fmt, stream):
+    """Enqueues the conversion of a bf16 ``[rows, cols]`` GPU tensor; ``_pack_weight_end`` checks it."""
     if fmt not in MATRIX_FORMATS:
         raise ValueError(f"matrix format must be one of {MATRIX_FORMATS}, got {fmt!r}")
     _check_device_tensor(w, "w", torch.bfloat16)
     if w.dim() != 2:
         raise ValueError("w must be 2-D")
-    if fmt in _MANTISSA_BITS:
-        q, e8 = _quantize(w, fmt, stream)
-        return pack_canonical(q, e8, fmt, strict=strict, stream=stream)
     rows, cols = w.shape
-    nbytes = _lib.lib().qmlp_packed_bytes(rows, cols, _lib.FMT_BF16)
+    code = _lib.FORMATS[fmt]
+    nbytes = _lib.lib().qmlp_packed_bytes(rows, cols, code)
     if nbytes == 0:
         raise ValueError(f"unsupported shape {rows}x{cols}: rows must be a multiple of 16 and cols of 256")
     buf = torch.empty(nbytes, dtype=torch.uint8, device=w.device)
-    _lib.check(_lib.lib().qmlp_pack(_lib.ptr(w), None, rows, cols, _lib.FMT_BF16, _lib.ptr(buf), nbytes,
-                                    _lib.stream_handle(stream)), "qmlp_pack")
-    return _read_info(PackedWeight(buf, rows, cols, "bf16"), stream)
+    _lib.check(_lib.lib().qmlp_quantize_pack(_lib.ptr(w), rows, cols, code, _lib.ptr(buf), nbytes,
+                                             _lib.stream_handle(stream)), "qmlp_quantize_pack")
+    return PackedWeight(buf, rows, cols, fmt)
+
+
+def _pack_weight_end(pw, strict, stream):
+    """Waits for the conversion and refuses non-finite values and, with ``strict``, flushed groups."""
+    norm = ctypes.c_double(0.0)
+    flushed, bad = ctypes.c_uint32(0), ctypes.c_uint32(0)
+    _lib.check(_lib.lib().qmlp_quantize_pack_info(_lib.ptr(pw.buf), pw.rows, pw.cols, pw.fmt_code, ctypes.byref(norm),
+                                                  ctypes.byref(flushed), ctypes.byref(bad),
+                                                  _lib.stream_handle(stream)), "qmlp_quantize_pack_info")
+    pw.max_row_norm = float(norm.value)
+    pw.flushed_groups = int(flushed.value)
+    if bad.value:
+        raise ValueError(f"weight holds non-finite values in {bad.value} groups")
+    if strict and pw.flushed_groups:
+        raise ValueError(f"{pw.flushed_groups} {pw.fmt} groups lie more than 19 binades below their row maximum")
+    return pw
+
+
+def pack_weight(w, fmt="bfp8", strict=True, stream=None):
+    """bf16 ``[rows, cols]`` GPU tensor (HF layout: [out, in]) -> PackedWeight in the matrix format
+    ``fmt`` ("bf16", "bfp8" or "bf4")."""
+    return _pack_weight_end(_pack_weight_begin(w, fmt, stream), strict, stream)
 
 
 def unpack_bfp8(pw, stream=None):
@@ -307,6 +326,14 @@ class MLPWeights:
         return self.w1.stream_bytes + self.w2.stream_bytes + self.w3.stream_bytes
 
 
+def _finish_load(pw, cache, strict):
+    _pack_weight_end(pw, strict, None)
+    if cache is not None:
+        from . import weight_cache
+
+        weight_cache.save(cache, pw)
+
+
 def load_mlp_weights(device, state_dict, tensor_cache_path=None, args=None, weight_format="bfp8", strict=True):
     """Per-layer MLP state -> MLPWeights (``mlp.py:45-169``).
 
@@ -323,7 +350,7 @@ def load_mlp_weights(device, state_dict, tensor_cache_path=None, args=None, weig
     if device.type != "cuda":
         raise ValueError(f"device must be a GPU, got {device}")
     names = {"w1": "gate_proj", "w2": "down_proj", "w3": "up_proj"}
-    packed = {}
+    packed, pending = {}, []  # a matrix's conversion is checked while the next one's runs
     for field, name in names.items():
         mfmt = down_fmt if field == "w2" else gu_fmt
         cache = None
@@ -352,12 +379,13 @@ def load_mlp_weights(device, state_dict, tensor_cache_path=None, args=None, weig
         if not isinstance(w, torch.Tensor):
             w = torch.as_tensor(w)
         w = w.to(device=device, dtype=torch.bfloat16).contiguous()
-        packed[field] = pack_weight(w, mfmt, strict=strict)
+        packed[field] = _pack_weight_begin(w, mfmt, None)
         del w
-        if cache is not None:
-            from . import weight_cache
-
-            weight_cache.save(cache, packed[field])
+        pending.append((packed[field], cache))
+        if len(pending) > 1:
+            _finish_load(*pending.pop(0), strict)
+    while pending:
+        _finish_load(*pending.pop(0), strict)
     weights = MLPWeights(**packed)
     I, H = weights.w1.rows, weights.w1.cols
     if (weights.w3.rows, weights.w3.cols) != (I, H) or (weights.w2.rows, weights.w2.cols) != (H, I):

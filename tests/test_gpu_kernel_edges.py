@@ -62,3 +62,42 @@ def test_non_finite_rows_stay_in_their_rows(pkg, cuda, fmt, M):
         assert torch.isfinite(good).all()
         assert torch.equal(got[keep], good[keep])
         assert not torch.isfinite(got[[2, 4]]).any()
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "bfp8", "bf4"])
+@pytest.mark.parametrize("rows,cols", [(16, 256), (48, 2048), (16, 2304), (32, 4352), (16, 45056), (16, 45312)])
+def test_quantize_pack_matches_the_separate_passes(pkg, cuda, fmt, rows, cols):
+    """The one-pass conversion writes the bytes of quantise + pack: fewer superblocks than waves, a
+    remainder, the longest row whose exponents wait in LDS and the shortest whose do not; any finite
+    bit pattern, denormals, ranges wide enough to flush groups, zero groups."""
+    import torch
+    from qwen_mlp_amd import _lib, mlp
+
+    g = torch.Generator(cuda).manual_seed(rows + cols)
+    normal = torch.randn(rows, cols, generator=g, device=cuda) * 0.02
+    anyv = torch.randint(-32768, 32768, (rows, cols), generator=g, device=cuda).to(torch.int16).view(torch.bfloat16)
+    binades = torch.randint(-30, 1, (rows, cols // 16), generator=g, device=cuda).float()
+    inputs = {
+        "any": torch.where(torch.isfinite(anyv.float()), anyv, torch.zeros_like(anyv)),
+        "normal": normal.bfloat16(),
+        "wide": (normal * torch.exp2(binades).repeat_interleave(16, dim=1)).bfloat16(),
+        "denormal": (normal.double() * 2.0 ** -126).bfloat16(),
+        "sparse": (normal * (torch.rand(rows, cols, generator=g, device=cuda) < 0.05)).bfloat16(),
+        "zero": torch.zeros_like(anyv),
+    }
+    for name, w in inputs.items():
+        got = mlp.pack_weight(w, fmt, strict=False)
+        if fmt == "bf16":
+            buf = torch.empty_like(got.buf)
+            _lib.check(_lib.lib().qmlp_pack(_lib.ptr(w), None, rows, cols, _lib.FMT_BF16, _lib.ptr(buf), buf.numel(),
+                                            _lib.stream_handle()), "qmlp_pack")
+        else:
+            want = mlp.pack_canonical(*mlp._quantize(w, fmt, None), fmt, strict=False)
+            buf = want.buf
+            assert (got.max_row_norm, got.flushed_groups) == (want.max_row_norm, want.flushed_groups), name
+        assert torch.equal(got.buf, buf), name
+    if fmt != "bf16":
+        w = inputs["normal"].clone()
+        w[rows - 1, 5], w[rows - 2, cols - 1] = float("nan"), float("-inf")
+        with pytest.raises(ValueError, match="non-finite values in 2 groups"):
+            mlp.pack_weight(w, fmt)
