@@ -221,6 +221,13 @@ int qmlp_set_profile_events(void* const* events, int n);
  * (scripts/ci/test_fused_1d.py:71-79). */
 int qmlp_plan_stream(int rows, int K, int num_cus, int* out2);
 
+/* Work split of the many-token kernel (M > 32) for one projection of an MLP of `fmt` weights (down
+ * != 0: the down projection, [H, I]; else the gate/up pair) on `num_cus` compute units.  Fills
+ * out[0..7] = {features per tile, tokens per tile, tiles, leading tiles that run whole, K pieces of
+ * each other tile (1: none is split), blocks launched, bytes of one piece's partial tile, bytes the
+ * workspace holds for the pieces}. */
+int qmlp_plan_tiles(int M, int H, int I, int fmt, int down, int num_cus, int* out8);
+
 /* Work split of the M <= 32 weight-streaming kernel for one projection with `nmat` matrices
  * (2 = gate/up, 1 = down) at M tokens (1..32; 17..32 run as two groups of 16): the (16-row tile
  * x 256-K superblock) grid cut into tile groups x K splits, split q covering superblocks

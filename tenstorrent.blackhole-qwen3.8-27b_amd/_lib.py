@@ -44,6 +44,7 @@ SIGNATURES = {
     "qmlp_forward_ex": (_I, [_P, _P, _P, _P, _P, _P, _P, _SZ, _I, _I, _I, _I, _I, _P]),
     "qmlp_workspace_bytes": (_SZ, [_I, _I, _I, _I]),
     "qmlp_workspace_init": (_I, [_P, _SZ, _P]),
+    "qmlp_plan_tiles": (_I, [_I, _I, _I, _I, _I, _I, ctypes.POINTER(ctypes.c_int)]),
     "qmlp_plan_stream": (_I, [_I, _I, _I, ctypes.POINTER(ctypes.c_int)]),
     "qmlp_set_profile_events": (_I, [_P, _I]),
     "qmlp_plan_split": (_I, [_I, _I, _I, _I, _I, ctypes.POINTER(ctypes.c_int)]),

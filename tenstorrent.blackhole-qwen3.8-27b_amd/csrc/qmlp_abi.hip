@@ -83,16 +83,15 @@ WsLayout ws_layout(int M, int H, int I, int fmt) {
   off = align256(off + std::max(sk_d, gv_d));
   L.pss = off;
   off = align256(off + (size_t)kMaxWorkgroups * 64 * 4);
-  // x16 and xn are read only by the gate/up projection; the many-token down projection reuses
-  // both (adjacent) for the partial tiles of its K-split tail.
   L.x16 = off;
   off = align256(off + (fmt != QMLP_FMT_BF16 ? (size_t)M * H * 2 : 0));
   L.xn = off;  // bf16 [M, H]: the normalised activations when the RMSNorm runs as its own pass
-  // The partial tiles of the many-token kernels' K-split pieces share xn's place: xn is read only
-  // before the gate/up projection (by the activation prep, or by gate/up itself for bf16 weights).
+  // The partial tiles of the many-token kernels' K-split pieces share xn's place with block-float
+  // weights, whose activation pass is xn's only reader; bf16 gate/up reads xn while it splits.
+  L.split_bytes = tiled_split_bytes(M);
+  if (fmt == QMLP_FMT_BF16) off = align256(off + (size_t)M * H * 2);
   L.split = off;
-  L.split_bytes = tiled_split_bytes(M, H, I, fmt);
-  off = align256(off + std::max((size_t)M * H * 2, L.split_bytes));
+  off = align256(off + std::max(fmt == QMLP_FMT_BF16 ? 0 : (size_t)M * H * 2, L.split_bytes));
   L.total = off;
   return L;
 }
@@ -379,6 +378,14 @@ int qmlp_plan_split(int rows, int K, int nmat, int M, int num_cus, int* out6) {
   out6[3] = p.KQ;
   out6[4] = p.Ng;
   out6[5] = p.maxseg;
+  return 0;
+}
+
+int qmlp_plan_tiles(int M, int H, int I, int fmt, int down, int num_cus, int* out8) {
+  if (!out8) return set_error(QMLP_E_NULL, "qmlp_plan_tiles: null pointer");
+  if (M <= 32 || M > 65536 || num_cus < 1 || !shape_ok(16, H) || !shape_ok(16, I) || !known_fmt(fmt))
+    return set_error(QMLP_E_SHAPE, "qmlp_plan_tiles: M=%d H=%d I=%d fmt=%d on %d CUs", M, H, I, fmt, num_cus);
+  plan_tiles_info(M, H, I, fmt, down != 0, num_cus, out8);
   return 0;
 }
 

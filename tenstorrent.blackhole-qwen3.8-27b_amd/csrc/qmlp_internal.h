@@ -110,10 +110,11 @@ int launch_prep(const ForwardArgs& a, hipStream_t s);
 int launch_rmsnorm(const void* x, const void* w, float eps, int M, int H, void* xn, hipStream_t s);
 int launch_forward_tiled(const ForwardArgs& a, int num_cus, hipStream_t s);
 bool tiled_supported(int M, int H, int I);
-// Workspace bytes for the partial tiles of the 32x32 many-token kernels' K-split pieces (0 where
-// neither projection of the shape splits on kSplitMaxSlots resident blocks).
+// Workspace bytes for the partial tiles of the many-token kernels' K-split pieces: kSplitMaxSlots of
+// the largest.
 constexpr int kSplitMaxSlots = 256;
-size_t tiled_split_bytes(int M, int H, int I, int fmt);
+size_t tiled_split_bytes(int M);
+void plan_tiles_info(int M, int H, int I, int fmt, bool down, int num_cus, int* out8);
 int launch_forward_gemv(const ForwardArgs& a, int num_cus, hipStream_t s);
 // Stream-K weight-streaming kernels for M <= 32 (qmlp_stream.hip).
 int plan_stream(int rows, int K, int num_cus, int* P, int* maxseg);

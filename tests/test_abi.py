@@ -204,6 +204,36 @@ def test_gemv_split_covers_every_unit_once(pkg, rows, K, nmat, M):
         assert all(c == 1 for row in covered for c in row)
 
 
+@pytest.mark.parametrize("fmt", [0, 1, 2])
+@pytest.mark.parametrize("H,I", [(5120, 17408), (5120, 8704), (1024, 3072), (256, 512), (16384, 256), (5376, 41728)])
+def test_tile_plans_cover_the_outputs_and_fit(pkg, H, I, fmt):
+    """M > 32 kernel: tiles of every height cover features x tokens once, no token block is wholly
+    padding, the whole tiles that lead come in whole rounds, pieces have at least one 64-K step,
+    their partial tiles fit the workspace region and their counters theirs."""
+    out = (ctypes.c_int * 8)()
+    heights = set()
+    for cus in (256, 304, 64, 1):
+        for M in (*range(33, 400), 777, 1024, 2047, 2048, 2049, 4100, 65536):
+            for down in (0, 1):
+                assert pkg.lib().qmlp_plan_tiles(M, H, I, fmt, down, cus, out) == 0
+                feats, toks, tiles, nfull, ks, blocks, piece, region = out
+                N, K = (H, I) if down else (I, H)
+                nbm = -(-M // toks)
+                assert toks % 32 == 0 and 64 <= toks <= 224 and (nbm - 1) * toks < M
+                assert N % feats == 0 and tiles == N // feats * nbm and 0 <= nfull <= tiles
+                heights.add((feats, toks, ks > 1))
+                if ks == 1:
+                    assert nfull == tiles == blocks
+                    continue
+                tail = tiles - nfull
+                assert tail > 0 and nfull % cus == 0 and 2 <= ks <= K // 64
+                assert blocks - nfull == ks * (tail if nfull else -(-tail // 8) * 8)
+                assert tail * ks * piece <= region and tail <= 65536
+    assert len(heights) > 3
+    for bad in ((32, H, I, fmt), (65537, H, I, fmt), (64, H, I + 128, fmt), (64, H, I, 3)):
+        assert pkg.lib().qmlp_plan_tiles(*bad, 0, 256, out) != 0
+
+
 def test_plan_split_rejects_bad_widths(pkg):
     out = (ctypes.c_int * 6)()
     assert pkg.lib().qmlp_plan_split(17408, 5120, 2, 0, 256, out) != 0

@@ -101,3 +101,41 @@ def test_quantize_pack_matches_the_separate_passes(pkg, cuda, fmt, rows, cols):
         w[rows - 1, 5], w[rows - 2, cols - 1] = float("nan"), float("-inf")
         with pytest.raises(ValueError, match="non-finite values in 2 groups"):
             mlp.pack_weight(w, fmt)
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "bfp8", "bf4"])
+@pytest.mark.parametrize("H,I,M", [(2048, 6144, M) for M in (33, 65, 97, 129, 161, 193, 225, 321, 385, 449, 577, 777, 1153)]
+                         + [(5120, 17408, M) for M in (97, 201, 321, 449, 705, 777, 1281)]
+                         + [(5376, 12288, 300), (256, 2560, 100), (2560, 256, 640)])
+def test_tile_heights_and_splits(pkg, cuda, fmt, H, I, M):
+    """Many-token tiles of every height with one live token row in the last block or a ragged one,
+    whole, split from the first tile on, and split behind whole rounds (a plan for every M: the
+    printed line); plain and behind the norm, twice (the arrival counters are left at zero)."""
+    import ctypes
+
+    import numpy as np
+    import torch
+    from qwen_mlp_amd import _lib, workloads
+
+    out = (ctypes.c_int * 8)()
+    for down in (0, 1):
+        assert pkg.lib().qmlp_plan_tiles(M, H, I, {"bf16": 0, "bfp8": 1, "bf4": 2}[fmt], down, 256, out) == 0
+        print(fmt, H, I, M, "down" if down else "gate/up", list(out)[:6], flush=True)
+    mlp, sd = _mlp(pkg, cuda, H, I, fmt, M)
+    x = workloads.activations(M, H, seed=80 + M, device=cuda)
+    nw = (torch.randn(H, generator=torch.Generator(cuda).manual_seed(5), device=cuda) * 0.1).to(torch.bfloat16)
+    y = mlp.forward(x, residual=x, out_dtype=torch.float32)
+    n = mlp.forward_rmsnorm(x, nw, out_dtype=torch.float32)
+    assert torch.equal(mlp.forward(x, residual=x, out_dtype=torch.float32), y)
+    assert torch.equal(mlp.forward(x, residual=x), y.to(torch.bfloat16))
+    assert torch.equal(mlp.forward_rmsnorm(x, nw, out_dtype=torch.float32), n)
+    torch.cuda.synchronize()
+    rows = np.unique(np.r_[np.arange(0, M, 61), np.arange(0, M, 32)[-3:], M - 1])
+    hw = host_weights(pkg, sd, fmt)
+    xf = x.float().cpu().numpy()[rows]
+    check(y.cpu().numpy()[rows],
+          omlp.swiglu(xf, hw["gate_proj"], hw["up_proj"], hw["down_proj"], residual=xf, h_bf16=fmt == "bf16"),
+          f"tiles {fmt} H={H} I={I} M={M}")
+    check(n.cpu().numpy()[rows],
+          omlp.norm_swiglu(xf, nw.float().cpu().numpy(), hw["gate_proj"], hw["up_proj"], hw["down_proj"], 1e-6),
+          f"tiles, norm {fmt} H={H} I={I} M={M}")
