@@ -21,8 +21,8 @@
 //
 // Epilogue (fp32 accumulators in registers): gate/up -> h = silu(g) * u rounded once (fp16 *
 // 2^th for block-float, bf16 for bf16 weights); down -> out = residual + y.  Every output element is
-// owned by one lane of one wave; a tile whose K range is split over a few blocks is finished by the
-// last of them, which adds their fp32 partial tiles in K order (deterministic).
+// owned by one lane of one wave; a tile whose K range is split over a few blocks is finished by a
+// second launch, which adds their fp32 partial tiles in K order (deterministic).
 #include <algorithm>
 #include <mutex>
 #include <set>
@@ -42,11 +42,10 @@ struct TlParams {
   int M, K, N, C;        // N output features, C = K / 256
   int nbm;               // token blocks
   int nfull;             // leading blocks that take one whole tile each
-  int ntail;             // tiles that follow, split in K (blocks of padding tiles beyond exit)
+  int ntail;             // tiles that follow, split in K
   int ks;                // K pieces per split tile
   float* part;           // fp32 partial tiles, [split tile][piece][the block's outputs]
   int part_bytes;
-  int* counters;         // arrival counter per split tile, left at zero
   const int* tsrc;       // block-float: per-token exponent of src
   const int* tout;       // block-float gate/up: h16 = h * 2^tout[m]
   void* out;             // gate/up: h [M, N] 16-bit; down: out [M, N] bf16 or fp32
@@ -102,14 +101,60 @@ struct Tl32Stage {
 // (dequantisation, LDS reads, vector memory return); with few tokens by the weights' arrival.
 //
 // Work (plan_tiles): blocks [0, nfull) each take one whole tile; blocks from nfull take K pieces of
-// the ntail tiles that follow (rounded up to whole XCDs where every tile splits: the padding
-// blocks exit at once): ks consecutive blocks share a tile, piece q covering 64-K steps
+// the ntail tiles that follow: ks consecutive blocks share a tile, piece q covering 64-K steps
 // [q S / ks, (q + 1) S / ks) of its S.  The whole tiles come in complete rounds of resident blocks
 // and the pieces start together as those rounds end, so the blocks reading one feature block's
-// weights read the same K range at the same time (L2 reuse).  A split tile's pieces meet through
-// the workspace by last arrival; no block ever waits for another, so the kernel cannot stall
+// weights read the same K range at the same time (L2 reuse).  The pieces leave their partial tiles
+// in the workspace for sum_kernel; no block ever waits for another, so the kernel cannot stall
 // whatever else holds the CUs (other streams, other processes).
 constexpr int kTlNWV = 8;  // waves per block
+
+// ---------------------------------------------------------------- outputs
+//
+// Four rows n .. n + 3 of token m, from the sums and their exponents (block-float weights).
+
+// h = silu(g) * u, rounded once; eg, eu: row minus token exponents, to: h's exponent
+template <int WF>
+__device__ __forceinline__ void put_h(const TlParams& p, int m, int n, f32x4 g, f32x4 u, const int (&eg)[4],
+                                      const int (&eu)[4], int to) {
+  uint16_t o[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    float gv = g[v], uv = u[v];
+    if constexpr (WF) {
+      gv = __builtin_amdgcn_ldexpf(gv, eg[v]);
+      uv = __builtin_amdgcn_ldexpf(uv, eu[v]);
+    }
+    const float hv = silu_mul(gv, uv);
+    o[v] = WF ? f32_to_f16_bits(__builtin_amdgcn_ldexpf(hv, to)) : f32_to_bf16(hv);
+  }
+  *(u32x2*)((uint16_t*)p.out + (size_t)m * p.N + n) =
+      u32x2{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
+}
+
+// The residual words of an output (bf16: the low two; fp32: all four; none: zero).
+__device__ __forceinline__ u32x4 get_residual(const TlParams& p, int m, int n) {
+  if (!p.residual) return u32x4{0u, 0u, 0u, 0u};
+  if (p.res_f32) return *(const u32x4*)((const float*)p.residual + (size_t)m * p.N + n);
+  const u32x2 w = *(const u32x2*)((const uint16_t*)p.residual + (size_t)m * p.N + n);
+  return u32x4{w.x, w.y, 0u, 0u};
+}
+
+// out = residual + y * 2^e
+template <int WF>
+__device__ __forceinline__ void put_out(const TlParams& p, int m, int n, f32x4 y, const int (&e)[4], u32x4 res) {
+  const f32x4 r = p.res_f32 ? __builtin_bit_cast(f32x4, res)
+                            : f32x4{bf16_to_f32((uint16_t)(res.x & 0xffffu)), bf16_to_f32((uint16_t)(res.x >> 16)),
+                                    bf16_to_f32((uint16_t)(res.y & 0xffffu)), bf16_to_f32((uint16_t)(res.y >> 16))};
+#pragma unroll
+  for (int v = 0; v < 4; ++v) y[v] = (WF ? __builtin_amdgcn_ldexpf(y[v], e[v]) : y[v]) + r[v];
+  if (p.out_f32) {
+    *(f32x4*)((float*)p.out + (size_t)m * p.N + n) = y;
+  } else {
+    const uint32_t o0 = f32_to_bf16(y[0]), o1 = f32_to_bf16(y[1]), o2 = f32_to_bf16(y[2]), o3 = f32_to_bf16(y[3]);
+    *(u32x2*)((uint16_t*)p.out + (size_t)m * p.N + n) = u32x2{o0 | (o1 << 16), o2 | (o3 << 16)};
+  }
+}
 
 enum { kDown = 0, kPair = 1, kBoth = 2 };
 
@@ -144,12 +189,9 @@ __global__ __launch_bounds__(512) void tiled32_kernel(TlParams p) {
   const bool full = (int)blockIdx.x < p.nfull;
   const int b = full ? (int)blockIdx.x : (int)blockIdx.x - p.nfull;
   const int ks = full ? 1 : p.ks;
-  // blocks sharing weights share an XCD (the pieces of a split tile too, where ks divides the
-  // part's blocks per XCD: their partial tiles then meet in one L2)
-  const int P = full ? p.nfull : (int)gridDim.x - p.nfull;
-  const int L = full || (P / 8) % ks == 0 ? xcd_logical(b, P) : b;
+  const int L = xcd_logical(b, full ? p.nfull : (int)gridDim.x - p.nfull);  // blocks sharing weights share an XCD
   const int tt = L / ks, q = L % ks;  // split tiles: index among them, piece
-  if (!full && tt >= p.ntail) return;  // a padding tile (the split tiles rounded up to whole XCDs)
+  if (!full && tt >= p.ntail) return;  // the pieces' rounding up to whole XCDs
   const int tile = full ? L : p.nfull + tt;
   const int bn = tile / p.nbm, bm = tile % p.nbm;
   const int m0 = bm * MG * 32;
@@ -370,70 +412,24 @@ __global__ __launch_bounds__(512) void tiled32_kernel(TlParams p) {
     });
   }
 
-  // A split tile is finished by last arrival: every piece publishes its whole partial tile in its
-  // slot (tt, q) with write-through stores, waits for them and counts itself; the piece whose
-  // count completes the tile (whichever it is) leaves the counter at zero and goes on with the
-  // sums of the ks partial tiles -- its own among them -- in K order, p_0 + p_1 + ... + p_{ks-1},
-  // which do not depend on the arrival order (deterministic).  No piece waits for another.
+  // A split tile's pieces leave their partial tiles in their slots (tt, q); sum_kernel, the next
+  // launch, adds them.
   auto own = [&](int mat, int g, int v4) {
     return f32x4{acc[mat][g][4 * v4], acc[mat][g][4 * v4 + 1], acc[mat][g][4 * v4 + 2], acc[mat][g][4 * v4 + 3]};
   };
-  const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(p.part, 0, p.part_bytes, kBufferRsrcWord3);
-  auto off = [&](int qq, int mat, int g, int v4) {  // byte offset of this lane's chunk in piece qq's slot
-    return (uint32_t)(tt * ks + qq) * PART_BYTES + (uint32_t)((((wave * NM + mat) * MG + g) * 4 + v4) * 64 + lane) * 16u;
-  };
   if (ks > 1) {
-    __shared__ int s_last;
+    const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(p.part, 0, p.part_bytes, kBufferRsrcWord3);
+    const uint32_t slot = (uint32_t)(tt * ks + q) * PART_BYTES + (uint32_t)(wave * NM * MG * 256 + lane) * 16u;
 #pragma unroll
     for (int mat = 0; mat < NM; ++mat)
 #pragma unroll
       for (int g = 0; g < MG; ++g)
 #pragma unroll
-        for (int v4 = 0; v4 < 4; ++v4) store_coherent(prs, off(q, mat, g, v4), own(mat, g, v4));
-    wait_stores();
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      const int old = __hip_atomic_fetch_add(p.counters + tt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      s_last = old == ks - 1;
-      if (s_last) __hip_atomic_store(p.counters + tt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
-    if (!s_last) return;
+        for (int v4 = 0; v4 < 4; ++v4)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, own(mat, g, v4)), prs,
+                                                 slot + (uint32_t)((mat * MG + g) * 4 + v4) * 1024u, 0, 0);
+    return;
   }
-  // The group's sums: the accumulators, or the ks partial tiles' chunks added in K order, RB
-  // pieces per round trip (offsets past the last piece lie beyond the descriptor's extent and read
-  // as zero without touching memory, so every load is unconditional).
-  auto sums = [&](int g, f32x4 (&a)[NM][4]) {
-    if (ks == 1) {
-#pragma unroll
-      for (int mat = 0; mat < NM; ++mat)
-#pragma unroll
-        for (int v4 = 0; v4 < 4; ++v4) a[mat][v4] = own(mat, g, v4);
-      return;
-    }
-    constexpr int RB = NM * MG > 6 ? 2 : 4;
-#pragma unroll
-    for (int mat = 0; mat < NM; ++mat)
-#pragma unroll
-      for (int v4 = 0; v4 < 4; ++v4) a[mat][v4] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int r0 = 0; r0 < ks; r0 += RB) {
-      f32x4 v[RB][NM][4];
-#pragma unroll
-      for (int r = 0; r < RB; ++r)
-#pragma unroll
-        for (int mat = 0; mat < NM; ++mat)
-#pragma unroll
-          for (int v4 = 0; v4 < 4; ++v4)
-            v[r][mat][v4] = load_coherent(prs, r0 + r < ks ? off(r0 + r, mat, g, v4) : 0xfffffff0u);
-#pragma unroll
-      for (int r = 0; r < RB; ++r)
-#pragma unroll
-        for (int mat = 0; mat < NM; ++mat)
-#pragma unroll
-          for (int v4 = 0; v4 < 4; ++v4) a[mat][v4] += v[r][mat][v4];
-    }
-  };
-
   // Epilogue, one group of 32 tokens at a time.  Accumulator v of lane l holds row
   // 8 (v / 4) + 4 (l / 32) + v % 4 of the wave's 32-row unit for token l % 32 of the group.
   const int col = lane & 31, rq = (lane >> 5) * 4;
@@ -447,58 +443,25 @@ __global__ __launch_bounds__(512) void tiled32_kernel(TlParams p) {
     constexpr int RG = MG < 4 ? MG : 4;
 #pragma unroll
     for (int g0 = 0; g0 < MG; g0 += RG) {
-      u32x4 rres[RG][4];  // bf16: the low two words; fp32: all four
+      u32x4 rres[RG][4];
 #pragma unroll
       for (int i = 0; i < RG; ++i)
 #pragma unroll
-        for (int vq = 0; vq < 4; ++vq) rres[i][vq] = u32x4{0u, 0u, 0u, 0u};
-      if (p.residual) {
-#pragma unroll
-        for (int i = 0; i < RG; ++i) {
-          const size_t row = (size_t)min(m0 + (g0 + i) * 32 + col, p.M - 1) * p.N;
-#pragma unroll
-          for (int vq = 0; vq < 4; ++vq) {
-            const int n = pair * 32 + vq * 8 + rq;
-            if (p.res_f32) {
-              rres[i][vq] = *(const u32x4*)((const float*)p.residual + row + n);
-            } else {
-              const u32x2 w = *(const u32x2*)((const uint16_t*)p.residual + row + n);
-              rres[i][vq] = u32x4{w.x, w.y, 0u, 0u};
-            }
-          }
-        }
-      }
+        for (int vq = 0; vq < 4; ++vq)
+          rres[i][vq] = get_residual(p, min(m0 + (g0 + i) * 32 + col, p.M - 1), pair * 32 + vq * 8 + rq);
 #pragma unroll
       for (int i = 0; i < RG; ++i) {
         const int g = g0 + i;
         if (g >= MG) break;
         const int m = m0 + g * 32 + col;
-        f32x4 a[NM][4];
-        sums(g, a);
         if (m >= p.M) continue;
         const int ts = WF ? ltok[32 * g] : 0;
-        f32x4 rr[4];
 #pragma unroll
         for (int vq = 0; vq < 4; ++vq) {
-          const u32x4 w = rres[i][vq];
-          rr[vq] = p.res_f32 ? __builtin_bit_cast(f32x4, w)
-                             : f32x4{bf16_to_f32((uint16_t)(w.x & 0xffffu)), bf16_to_f32((uint16_t)(w.x >> 16)),
-                                     bf16_to_f32((uint16_t)(w.y & 0xffffu)), bf16_to_f32((uint16_t)(w.y >> 16))};
-        }
+          int e[4];
 #pragma unroll
-        for (int vq = 0; vq < 4; ++vq) {
-          const int n = pair * 32 + vq * 8 + rq;
-          float y[4];
-#pragma unroll
-          for (int v = 0; v < 4; ++v)
-            y[v] = (WF ? __builtin_amdgcn_ldexpf(a[0][vq][v], lrow[8 * vq + v] - ts) : a[0][vq][v]) + rr[vq][v];
-          if (p.out_f32) {
-            *(f32x4*)((float*)p.out + (size_t)m * p.N + n) = f32x4{y[0], y[1], y[2], y[3]};
-          } else {
-            const uint32_t o0 = f32_to_bf16(y[0]), o1 = f32_to_bf16(y[1]), o2 = f32_to_bf16(y[2]),
-                           o3 = f32_to_bf16(y[3]);
-            *(u32x2*)((uint16_t*)p.out + (size_t)m * p.N + n) = u32x2{o0 | (o1 << 16), o2 | (o3 << 16)};
-          }
+          for (int v = 0; v < 4; ++v) e[v] = WF ? lrow[8 * vq + v] - ts : 0;
+          put_out<WF>(p, m, pair * 32 + vq * 8 + rq, own(0, g, vq), e, rres[i][vq]);
         }
       }
     }
@@ -510,27 +473,23 @@ __global__ __launch_bounds__(512) void tiled32_kernel(TlParams p) {
       const int ts = WF ? ltok[32 * g] : 0, to = WF ? ltok[MG * 32 + 32 * g] : 0;
 #pragma unroll
       for (int vq = 0; vq < 4; ++vq) {
-        const int n = pair * 32 + vq * 8 + rq;
-        uint16_t o[4];
+        int eg[4], eu[4];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          float gv = gate[vq][v], uv = up[vq][v];
-          if constexpr (WF) {
-            gv = __builtin_amdgcn_ldexpf(gv, lrow[8 * vq + v] - ts);
-            uv = __builtin_amdgcn_ldexpf(uv, lrow[UNITS * 32 + 8 * vq + v] - ts);
-          }
-          const float hv = silu_mul(gv, uv);
-          o[v] = WF ? f32_to_f16_bits(__builtin_amdgcn_ldexpf(hv, to)) : f32_to_bf16(hv);
+          eg[v] = WF ? lrow[8 * vq + v] - ts : 0;
+          eu[v] = WF ? lrow[UNITS * 32 + 8 * vq + v] - ts : 0;
         }
-        *(u32x2*)((uint16_t*)p.out + (size_t)m * p.N + n) =
-            u32x2{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
+        put_h<WF>(p, m, pair * 32 + vq * 8 + rq, gate[vq], up[vq], eg, eu, to);
       }
     };
     if constexpr (MODE == kBoth) {
 #pragma unroll
       for (int g = 0; g < MG; ++g) {
         f32x4 a[NM][4];
-        sums(g, a);
+#pragma unroll
+        for (int mat = 0; mat < NM; ++mat)
+#pragma unroll
+          for (int vq = 0; vq < 4; ++vq) a[mat][vq] = own(mat, g, vq);
         finish(g, a[0], a[NM - 1]);
       }
     } else {
@@ -540,23 +499,92 @@ __global__ __launch_bounds__(512) void tiled32_kernel(TlParams p) {
 #pragma unroll
       for (int g0 = 0; g0 < MG; g0 += 2) {
         f32x4* buf = (f32x4*)(lds + (size_t)(g0 & 2) / 2 * kSwapBytes) + lane;
-        f32x4 a0[NM][4], a1[NM][4], o[4];
-        sums(g0, a0);
-        if (g0 + 1 < MG) sums(g0 + 1 < MG ? g0 + 1 : g0, a1);
+        f32x4 a0[4], a1[4], o[4];
 #pragma unroll
-        for (int vq = 0; vq < 4; ++vq)
-          if (up || g0 + 1 < MG) buf[(wave * 4 + vq) * 64] = up ? a0[0][vq] : a1[0][vq];
+        for (int vq = 0; vq < 4; ++vq) {
+          a0[vq] = own(0, g0, vq);
+          a1[vq] = own(0, g0 + 1 < MG ? g0 + 1 : g0, vq);
+          if (up || g0 + 1 < MG) buf[(wave * 4 + vq) * 64] = up ? a0[vq] : a1[vq];
+        }
         __syncthreads();
         if (up && g0 + 1 >= MG) continue;
 #pragma unroll
         for (int vq = 0; vq < 4; ++vq) o[vq] = buf[((wave ^ UNITS) * 4 + vq) * 64];
         if (up)
-          finish(g0 + 1, o, a1[0]);
+          finish(g0 + 1, o, a1);
         else
-          finish(g0, a0[0], o);
+          finish(g0, a0, o);
       }
     }
   }
+}
+
+// Adds the ks partial tiles of each split tile in K order and finishes its outputs: a block per
+// (split tile, 32-row unit, group of 32 tokens), a wave per 8 rows, the lanes as in the tile's
+// accumulators.  Bound by reading the partial tiles (once, every CU taking part); KB of them are
+// requested at once, slots past the last piece beyond the descriptor's extent (they read as zero
+// without touching memory), so every load is unconditional.
+//
+// As a launch of its own it costs its start, ~4 us, and needs no arrival counter, no wait for
+// stores at the device level and no lone CU that adds a tile's pieces at the end: the last of a
+// tile's blocks used to read all ks partial tiles.
+template <int WF, int MODE>
+__global__ __launch_bounds__(256) void sum_kernel(TlParams p, int mg) {
+  constexpr int KB = 4, NM = MODE == kDown ? 1 : 2, UNITS = MODE == kPair ? 4 : 8;
+  const int lane = threadIdx.x & 63, vq = threadIdx.x >> 6;
+  const int g = blockIdx.x % mg, unit = blockIdx.x / mg % UNITS, tt = blockIdx.x / mg / UNITS;
+  const int tile = p.nfull + tt, bn = tile / p.nbm, bm = tile % p.nbm;
+  const int mr = (bm * mg + g) * 32 + (lane & 31), m = min(mr, p.M - 1);
+  const int n = (bn * UNITS + unit) * 32 + vq * 8 + (lane >> 5) * 4;
+  const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(p.part, 0, p.part_bytes, kBufferRsrcWord3);
+  // a piece's slot: [wave][matrix of the wave][group][vq][lane]
+  const uint32_t piece = (uint32_t)(kTlNWV * (MODE == kBoth ? 2 : 1) * mg) * 4096u;
+  uint32_t off[NM];
+#pragma unroll
+  for (int mat = 0; mat < NM; ++mat) {
+    const int w = MODE == kPair ? unit + mat * UNITS : unit, mw = MODE == kBoth ? mat : 0;
+    off[mat] = (uint32_t)(tt * p.ks) * piece +
+               (uint32_t)((((w * (MODE == kBoth ? 2 : 1) + mw) * mg + g) * 4 + vq) * 64 + lane) * 16u;
+  }
+  int er[NM][4], ts = 0, to = 0;
+  u32x4 res = u32x4{0u, 0u, 0u, 0u};
+  if constexpr (WF != 0) {
+#pragma unroll
+    for (int mat = 0; mat < NM; ++mat) {
+      const u32x4 e = *(const u32x4*)((mat ? p.rowexp1 : p.rowexp0) + n);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) er[mat][v] = (int)e[v];
+    }
+    ts = p.tsrc[m];
+    if constexpr (MODE != kDown) to = p.tout[m];
+  }
+  if constexpr (MODE == kDown) res = get_residual(p, m, n);
+  f32x4 sum[NM];
+#pragma unroll
+  for (int mat = 0; mat < NM; ++mat) sum[mat] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int r0 = 0; r0 < p.ks; r0 += KB) {
+    f32x4 v[KB][NM];
+#pragma unroll
+    for (int r = 0; r < KB; ++r)
+#pragma unroll
+      for (int mat = 0; mat < NM; ++mat)
+        v[r][mat] = __builtin_bit_cast(
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                       prs, r0 + r < p.ks ? off[mat] + (uint32_t)(r0 + r) * piece : 0xfffffff0u, 0, 0));
+#pragma unroll
+    for (int r = 0; r < KB; ++r)
+#pragma unroll
+      for (int mat = 0; mat < NM; ++mat) sum[mat] += v[r][mat];
+  }
+  if (mr >= p.M) return;
+#pragma unroll
+  for (int mat = 0; mat < NM; ++mat)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) er[mat][v] = WF ? er[mat][v] - ts : 0;
+  if constexpr (MODE == kDown)
+    put_out<WF>(p, m, n, sum[0], er[0], res);
+  else
+    put_h<WF>(p, m, n, sum[0], sum[NM - 1], er[0], er[NM - 1], to);
 }
 
 // ---------------------------------------------------------------- host side
@@ -566,32 +594,32 @@ __global__ __launch_bounds__(512) void tiled32_kernel(TlParams p) {
 // 4 % rms with the points near the fastest weighted most.
 struct TileCost {
   float step[8];   // one 64-K step of a tile of MG groups (0: height not built)
-  float tile;      // a whole tile's start and epilogue
+  float tile;      // a tile's, or a piece's, start and end
   float launch;    // the launch's
   float tbps;      // TB/s at which weights nobody shares arrive
-  float publish;   // publishing one group of one piece's matrix, spread over the CUs
-  float add;       // adding one group of one piece's matrix in a last arrival
-  float split;     // a split's fixed cost
+  float publish;   // writing and reading one group of one piece's matrix, spread over the CUs
+  float add;       // one more piece in the sums of one group of one matrix
+  float split;     // the second launch
+  float cold;      // what a step takes longer where one token block reads every weight
 };
-constexpr TileCost kCostPair{{0, 0, .49f, .75f, .91f, 1.17f, 1.32f, 1.53f}, 0.4f, 0.3f, 4.0f, .010f, .38f, 0.0f};
-constexpr TileCost kCostBoth{{0, 0, .95f, 0, 1.56f, 0, 0, 0}, 4.7f, 0.0f, 7.7f, .009f, .27f, 2.7f};
-constexpr TileCost kCostDown{{0, 0, .53f, .71f, .90f, 1.13f, 1.31f, 1.55f}, 7.3f, 0.0f, 7.6f, .006f, .80f, 4.5f};
-constexpr TileCost kCostPair16{{0, 0, .54f, .74f, .87f, 1.07f, 1.22f, 1.41f}, 5.3f, 17.5f, 6.7f, .003f, .32f, 0.8f};
-constexpr TileCost kCostDown16{{0, 0, .55f, .69f, .83f, 1.02f, 1.17f, 1.37f}, 13.7f, 9.1f, 11.4f, .004f, .83f, 0.0f};
-constexpr float kCold = 0.1f;  // us a step takes longer where one token block reads every weight
+constexpr TileCost kCostPair8{{0, 0, .49f, .74f, .92f, 1.15f, 1.33f, 1.55f}, 0.0f, 4.5f, 7.9f, .006f, .03f, 11.5f, .08f};
+constexpr TileCost kCostPair4{{0, 0, .48f, .65f, .89f, 1.20f, 1.30f, 1.51f}, 0.9f, 4.0f, 7.3f, .007f, .07f, 3.7f, .01f};
+constexpr TileCost kCostPair16{{0, 0, .57f, .78f, .92f, 1.13f, 1.26f, 1.46f}, 4.9f, 6.7f, 5.6f, .000f, .16f, 6.3f, .10f};
+constexpr TileCost kCostBoth{{0, 0, .98f, 0, 1.63f, 0, 0, 0}, 3.2f, 0.0f, 7.3f, .009f, .04f, 3.1f, .09f};
+constexpr TileCost kCostDown8{{0, 0, .53f, .74f, .93f, 1.16f, 1.36f, 1.61f}, 3.1f, 3.9f, 5.7f, .005f, .08f, 4.7f, .00f};
+constexpr TileCost kCostDown16{{0, 0, .55f, .73f, .87f, 1.07f, 1.20f, 1.40f}, 5.9f, 6.1f, 7.9f, .006f, .05f, 6.0f, .09f};
 
 // Largest K split of a tile, and how many rounds its pieces may take.
-constexpr int kMaxKs = 10, kMaxSplitRounds = 4;
+constexpr int kMaxKs = 12, kMaxSplitRounds = 4;
 
 // Bytes of one K piece's partial tile (8 waves x nm 32-row units x mg groups of 32 tokens, fp32).
 constexpr size_t split_part_bytes(int nm, int mg) { return (size_t)kTlNWV * nm * mg * 16 * 64 * 4; }
 
 // Work of one projection: `nfull` whole tiles, then the remaining ntail tiles in ks pieces of their
-// K range each (npad: ntail rounded up to whole XCDs where no whole tile leads; padding blocks
-// exit at once).
+// K range each.
 struct TilePlan {
   int mode, mg;
-  int nbm, nfull, ntail, ks, npad;
+  int nbm, nfull, ntail, ks;
   float cost;
 };
 
@@ -612,17 +640,17 @@ static void plan_mode(int mode, const TileCost& c, int M, int N, int C, int fmt,
     const int nbm = (M + mg * 32 - 1) / (mg * 32), T = nbn * nbm;
     // step(a): with a blocks at work, their distinct weights come from memory
     auto step = [&](int a) {
-      return std::max(c.step[mg], (float)a / (float)nbm * step_mb / c.tbps) + (nbm == 1 ? kCold : 0.f);
+      return std::max(c.step[mg] + (nbm == 1 ? c.cold : 0.f), (float)a / (float)nbm * step_mb / c.tbps);
     };
     const float full = (float)kst * step(slots) + c.tile;  // a round of whole tiles
     auto whole = [&](int n) {
       const int rest = n % slots;
       return (float)(n / slots) * full + (rest ? (float)kst * step(std::max(rest, nbm)) + c.tile : 0.f);
     };
-    auto take = [&](int nfull, int ntail, int ks, int npad, float cost) {
-      if (cost < best->cost) *best = {mode, mg, nbm, nfull, ntail, ks, npad, cost};
+    auto take = [&](int nfull, int ntail, int ks, float cost) {
+      if (cost < best->cost) *best = {mode, mg, nbm, nfull, ntail, ks, cost};
     };
-    take(T, 0, 1, 0, c.launch + whole(T));
+    take(T, 0, 1, c.launch + whole(T));
     for (int lead = 0; lead < 2; ++lead) {
       const int nfull = lead ? T / slots * slots : 0, ntail = T - nfull;
       if (ntail == 0 || (lead && nfull == 0)) continue;
@@ -631,7 +659,7 @@ static void plan_mode(int mode, const TileCost& c, int M, int N, int C, int fmt,
         if (P > (long long)kMaxSplitRounds * slots || (size_t)P * split_part_bytes(nm, mg) > part_bytes) break;
         const int rounds = ((int)P + slots - 1) / slots;
         const float groups = (float)(mg * nm);
-        take(nfull, ntail, ks, nfull ? ntail : (ntail + 7) / 8 * 8,
+        take(nfull, ntail, ks,
              c.launch + whole(nfull) +
                  (float)rounds * ((float)((kst + ks - 1) / ks) * step(std::min((int)P, slots)) + c.tile) + c.split +
                  (float)P * groups * c.publish + (float)ks * groups * c.add);
@@ -645,9 +673,9 @@ static TilePlan plan_tiles(bool down, int M, int N, int C, int fmt, int slots, s
   best.cost = 1e30f;
   slots = std::max(slots, 1);
   if (down) {
-    plan_mode(kDown, fmt ? kCostDown : kCostDown16, M, N, C, fmt, slots, part_bytes, &best);
+    plan_mode(kDown, fmt ? kCostDown8 : kCostDown16, M, N, C, fmt, slots, part_bytes, &best);
   } else {
-    plan_mode(kPair, fmt ? kCostPair : kCostPair16, M, N, C, fmt, slots, part_bytes, &best);
+    plan_mode(kPair, fmt == 2 ? kCostPair4 : fmt ? kCostPair8 : kCostPair16, M, N, C, fmt, slots, part_bytes, &best);
     if (fmt) plan_mode(kBoth, kCostBoth, M, N, C, fmt, slots, part_bytes, &best);
   }
   return best;
@@ -656,6 +684,10 @@ static TilePlan plan_tiles(bool down, int M, int N, int C, int fmt, int slots, s
 // Sized for the most any plan uses (plan_mode bounds its pieces by it): constant in M, so that the
 // workspace never shrinks as M grows.
 size_t tiled_split_bytes(int M) { return M <= 32 ? 0 : (size_t)kSplitMaxSlots * split_part_bytes(2, 4); }
+
+// Blocks of a plan's launch: the pieces rounded up to whole XCDs, so that consecutive ones share
+// an XCD (at most 7 exit at once).
+static int tile_blocks(const TilePlan& t) { return t.nfull + (t.ks > 1 ? (t.ntail * t.ks + 7) / 8 * 8 : 0); }
 
 void plan_tiles_info(int M, int H, int I, int fmt, bool down, int num_cus, int* out8) {
   const size_t bytes = tiled_split_bytes(M);
@@ -666,7 +698,7 @@ void plan_tiles_info(int M, int H, int I, int fmt, bool down, int num_cus, int* 
   out8[2] = t.nfull + t.ntail;
   out8[3] = t.nfull;
   out8[4] = t.ks;
-  out8[5] = t.nfull + t.npad * t.ks;
+  out8[5] = tile_blocks(t);
   out8[6] = (int)split_part_bytes(t.mode == kBoth ? 2 : 1, t.mg);
   out8[7] = (int)bytes;
 }
@@ -699,8 +731,12 @@ static int launch_tiled32(TlParams p, const TilePlan& t, hipStream_t s) {
   p.nfull = t.nfull;
   p.ntail = t.ntail;
   p.ks = t.ks;
-  launch_timed(MODE == kDown ? 1 : 0, kern, dim3(t.nfull + t.npad * t.ks), dim3(kTlNWV * 64), lds, s, p);
-  return check_launch("tiled32_kernel");
+  constexpr int slot = MODE == kDown ? 1 : 0;
+  launch_timed_part(slot, t.ks > 1 ? 1 : 3, kern, dim3(tile_blocks(t)), dim3(kTlNWV * 64), lds, s, p);
+  if (int rc = check_launch("tiled32_kernel")) return rc;
+  if (t.ks == 1) return 0;
+  launch_timed_part(slot, 2, sum_kernel<WF, MODE>, dim3(t.ntail * (MODE == kPair ? 4 : 8) * MG), dim3(256), 0, s, p, MG);
+  return check_launch("sum_kernel");
 }
 
 template <int WF, int MODE>
@@ -748,7 +784,6 @@ int launch_forward_tiled(const ForwardArgs& a, int num_cus, hipStream_t s) {
   g.out = h;
   g.part = (float*)(a.ws + L.split);
   g.part_bytes = (int)std::min<size_t>(L.split_bytes, (size_t)1 << 30);
-  g.counters = (int*)(a.ws + L.counters_gu);
   const TilePlan tg = plan_tiles(false, a.M, a.I, g.C, fmt, num_cus, (size_t)g.part_bytes);
   int rc;
   if (tg.mode == kBoth)
@@ -774,7 +809,6 @@ int launch_forward_tiled(const ForwardArgs& a, int num_cus, hipStream_t s) {
   d.res_f32 = a.res_f32;
   d.part = g.part;
   d.part_bytes = g.part_bytes;
-  d.counters = (int*)(a.ws + L.counters_d);
   const TilePlan td = plan_tiles(true, a.M, a.H, d.C, dfmt, num_cus, (size_t)d.part_bytes);
   return dfmt == 1 ? launch_mode<1, kDown>(d, td, s) : launch_mode<0, kDown>(d, td, s);
 }

@@ -209,7 +209,7 @@ def test_gemv_split_covers_every_unit_once(pkg, rows, K, nmat, M):
 def test_tile_plans_cover_the_outputs_and_fit(pkg, H, I, fmt):
     """M > 32 kernel: tiles of every height cover features x tokens once, no token block is wholly
     padding, the whole tiles that lead come in whole rounds, pieces have at least one 64-K step,
-    their partial tiles fit the workspace region and their counters theirs."""
+    their partial tiles fit the workspace region."""
     out = (ctypes.c_int * 8)()
     heights = set()
     for cus in (256, 304, 64, 1):
@@ -227,8 +227,8 @@ def test_tile_plans_cover_the_outputs_and_fit(pkg, H, I, fmt):
                     continue
                 tail = tiles - nfull
                 assert tail > 0 and nfull % cus == 0 and 2 <= ks <= K // 64
-                assert blocks - nfull == ks * (tail if nfull else -(-tail // 8) * 8)
-                assert tail * ks * piece <= region and tail <= 65536
+                assert blocks - nfull == -(-tail * ks // 8) * 8
+                assert tail * ks * piece <= region
     assert len(heights) > 3
     for bad in ((32, H, I, fmt), (65537, H, I, fmt), (64, H, I + 128, fmt), (64, H, I, 3)):
         assert pkg.lib().qmlp_plan_tiles(*bad, 0, 256, out) != 0

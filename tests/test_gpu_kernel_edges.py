@@ -110,7 +110,7 @@ def test_quantize_pack_matches_the_separate_passes(pkg, cuda, fmt, rows, cols):
 def test_tile_heights_and_splits(pkg, cuda, fmt, H, I, M):
     """Many-token tiles of every height with one live token row in the last block or a ragged one,
     whole, split from the first tile on, and split behind whole rounds (a plan for every M: the
-    printed line); plain and behind the norm, twice (the arrival counters are left at zero)."""
+    printed line); plain and behind the norm, twice."""
     import ctypes
 
     import numpy as np
