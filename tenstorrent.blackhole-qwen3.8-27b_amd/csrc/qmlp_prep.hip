@@ -114,8 +114,19 @@ __global__ __launch_bounds__(kRowThreads) void rows_kernel(const uint16_t* __res
       }
       ss += (double)cs;
     });
-    mx = row_reduce(mx, s_max, [](float a, float b) { return fmaxf(a, b); });
-    ss = row_reduce(ss, s_sum, [](double a, double b) { return a + b; });
+    // both reductions behind one barrier
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      mx = fmaxf(mx, __shfl_xor(mx, o));
+      ss += __shfl_xor(ss, o);
+    }
+    if ((tid & 63) == 0) {
+      s_max[tid >> 6] = mx;
+      s_sum[tid >> 6] = ss;
+    }
+    __syncthreads();
+    mx = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
+    ss = (s_sum[0] + s_sum[1]) + (s_sum[2] + s_sum[3]);
     int e = 0;
     if (mx > 0.f) frexpf(mx, &e);
     const int txm = mx > 0.f ? 15 - e : 0;

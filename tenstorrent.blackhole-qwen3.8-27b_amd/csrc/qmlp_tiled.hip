@@ -168,7 +168,7 @@ constexpr size_t tiled32_lds(int MG, int MODE) {
   return tiled32_exp_offset(MG, MODE) + (size_t)((MODE == kBoth ? 512 : 256) + (MODE == kDown ? 1 : 2) * MG * 32) * 4;
 }
 
-template <int WF, int MG, int NBB, int MODE>
+template <int WF, int MG, int NBB, int MODE, bool ONCE>
 __global__ __launch_bounds__(512) void tiled32_kernel(TlParams p) {
   constexpr int NWV = kTlNWV, NT = NWV * 64;
   constexpr int NM = MODE == kBoth ? 2 : 1;       // matrices of one wave
@@ -262,6 +262,10 @@ __global__ __launch_bounds__(512) void tiled32_kernel(TlParams p) {
         2 * tile_bytes, kBufferRsrcWord3);
   const uint32_t lp0 = (uint32_t)(32 * hk + (lane & 15)), lp1 = lp0 + 16u;
   const uint32_t wv = (uint32_t)((lane >> 4) & 1) * (uint32_t)tile_bytes;  // the lane's tile
+  // Weights that several token blocks read stay in L2 for them; with one token block (ONCE) they are
+  // read once and pass it by (27B layer at 64 tokens: bf16 127.4 -> 121.8 us, bfp8 82.4 -> 81.4; with
+  // several token blocks 1-6 % slower).
+  constexpr int POL = ONCE ? 2 : 0;  // buffer cache policy: non-temporal
   auto wload = [&](Tl32Stage<WF, NM>& st, int step) {
     const int sc = kb + min(step, nst - 1);
     const int bo = (sc >> 2) * BLK;
@@ -269,18 +273,18 @@ __global__ __launch_bounds__(512) void tiled32_kernel(TlParams p) {
     for (int mat = 0; mat < NM; ++mat) {
       if constexpr (WF == 1) {
         const int so = bo + (sc & 3) * 1024;
-        st.w[mat][0] = __builtin_amdgcn_raw_buffer_load_b128(wr[mat], wv + lp0 * 16u, so, 0);
-        st.w[mat][1] = __builtin_amdgcn_raw_buffer_load_b128(wr[mat], wv + lp1 * 16u, so, 0);
+        st.w[mat][0] = __builtin_amdgcn_raw_buffer_load_b128(wr[mat], wv + lp0 * 16u, so, POL);
+        st.w[mat][1] = __builtin_amdgcn_raw_buffer_load_b128(wr[mat], wv + lp1 * 16u, so, POL);
       } else if constexpr (WF == 2) {
         const int so = bo + (sc & 2) * 512 + (sc & 1) * 8;
         st.w[mat][0] = __builtin_amdgcn_raw_buffer_load_b64(wr[mat], wv + lp0 * 16u, so, 0);
         st.w[mat][1] = __builtin_amdgcn_raw_buffer_load_b64(wr[mat], wv + lp1 * 16u, so, 0);
       } else {
         const int so = bo + (sc & 3) * 2048;
-        st.w[mat][0] = __builtin_amdgcn_raw_buffer_load_b128(wr[mat], wv + lp0 * 16u, so, 0);
-        st.w[mat][1] = __builtin_amdgcn_raw_buffer_load_b128(wr[mat], wv + 1024u + lp0 * 16u, so, 0);
-        st.w[mat][2] = __builtin_amdgcn_raw_buffer_load_b128(wr[mat], wv + lp1 * 16u, so, 0);
-        st.w[mat][3] = __builtin_amdgcn_raw_buffer_load_b128(wr[mat], wv + 1024u + lp1 * 16u, so, 0);
+        st.w[mat][0] = __builtin_amdgcn_raw_buffer_load_b128(wr[mat], wv + lp0 * 16u, so, POL);
+        st.w[mat][1] = __builtin_amdgcn_raw_buffer_load_b128(wr[mat], wv + 1024u + lp0 * 16u, so, POL);
+        st.w[mat][2] = __builtin_amdgcn_raw_buffer_load_b128(wr[mat], wv + lp1 * 16u, so, POL);
+        st.w[mat][3] = __builtin_amdgcn_raw_buffer_load_b128(wr[mat], wv + 1024u + lp1 * 16u, so, POL);
       }
     }
   };
@@ -602,11 +606,11 @@ struct TileCost {
   float split;     // the second launch
   float cold;      // what a step takes longer where one token block reads every weight
 };
-constexpr TileCost kCostPair8{{0, 0, .49f, .74f, .92f, 1.15f, 1.33f, 1.55f}, 0.0f, 4.5f, 7.9f, .006f, .03f, 11.5f, .08f};
+constexpr TileCost kCostPair8{{0, 0, .53f, .75f, .92f, 1.15f, 1.33f, 1.55f}, 1.5f, 4.5f, 7.9f, .006f, .03f, 8.0f, .08f};
 constexpr TileCost kCostPair4{{0, 0, .48f, .65f, .89f, 1.20f, 1.30f, 1.51f}, 0.9f, 4.0f, 7.3f, .007f, .07f, 3.7f, .01f};
 constexpr TileCost kCostPair16{{0, 0, .57f, .78f, .92f, 1.13f, 1.26f, 1.46f}, 4.9f, 6.7f, 5.6f, .000f, .16f, 6.3f, .10f};
-constexpr TileCost kCostBoth{{0, 0, .98f, 0, 1.63f, 0, 0, 0}, 3.2f, 0.0f, 7.3f, .009f, .04f, 3.1f, .09f};
-constexpr TileCost kCostDown8{{0, 0, .53f, .74f, .93f, 1.16f, 1.36f, 1.61f}, 3.1f, 3.9f, 5.7f, .005f, .08f, 4.7f, .00f};
+constexpr TileCost kCostBoth{{0, 0, 1.02f, 0, 1.60f, 0, 0, 0}, 3.2f, 0.0f, 7.3f, .009f, .04f, 3.1f, .09f};
+constexpr TileCost kCostDown8{{0, 0, .53f, .75f, .93f, 1.16f, 1.36f, 1.61f}, 3.1f, 3.9f, 5.7f, .005f, .08f, 4.7f, .00f};
 constexpr TileCost kCostDown16{{0, 0, .55f, .73f, .87f, 1.07f, 1.20f, 1.40f}, 5.9f, 6.1f, 7.9f, .006f, .05f, 6.0f, .09f};
 
 // Largest K split of a tile, and how many rounds its pieces may take.
@@ -717,13 +721,13 @@ static int raise_lds_limit(const void* kern, size_t lds) {
   return 0;
 }
 
-template <int WF, int MODE, int MG>
+template <int WF, int MODE, int MG, bool ONCE>
 static int launch_tiled32(TlParams p, const TilePlan& t, hipStream_t s) {
   // B register buffers: three where the registers allow them; two for tall tiles, and for the bfp8
   // gate/up pair in one wave (three: 749 against 709-714 us at 2048 tokens, the compiler then waits
   // for every LDS read before its products).
   constexpr int NBB = MG >= 6 || (WF == 1 && MODE == kBoth) ? 2 : 3;
-  auto kern = tiled32_kernel<WF, MG, NBB, MODE>;
+  auto kern = tiled32_kernel<WF, MG, NBB, MODE, ONCE>;
   constexpr size_t lds = tiled32_lds(MG, MODE);
   if (lds > 64 * 1024)
     if (int rc = raise_lds_limit((const void*)kern, lds)) return rc;
@@ -739,18 +743,27 @@ static int launch_tiled32(TlParams p, const TilePlan& t, hipStream_t s) {
   return check_launch("sum_kernel");
 }
 
+// Weights one token block reads pass the L2 by only where a load takes whole 16-byte pieces: bf4's
+// 8-byte loads of two steps share their lines (64 tokens: 85.9 against 80.7 us).
+template <int WF, int MODE, int MG>
+static int launch_height(const TlParams& p, const TilePlan& t, hipStream_t s) {
+  if constexpr (WF != 2 && MG <= 3)
+    if (t.nbm == 1) return launch_tiled32<WF, MODE, MG, true>(p, t, s);
+  return launch_tiled32<WF, MODE, MG, false>(p, t, s);
+}
+
 template <int WF, int MODE>
 static int launch_mode(const TlParams& p, const TilePlan& t, hipStream_t s) {
   if constexpr (MODE == kBoth) {
-    return t.mg == 2 ? launch_tiled32<WF, MODE, 2>(p, t, s) : launch_tiled32<WF, MODE, 4>(p, t, s);
+    return t.mg == 2 ? launch_height<WF, MODE, 2>(p, t, s) : launch_height<WF, MODE, 4>(p, t, s);
   } else {
     switch (t.mg) {
-      case 2: return launch_tiled32<WF, MODE, 2>(p, t, s);
-      case 3: return launch_tiled32<WF, MODE, 3>(p, t, s);
-      case 4: return launch_tiled32<WF, MODE, 4>(p, t, s);
-      case 5: return launch_tiled32<WF, MODE, 5>(p, t, s);
-      case 6: return launch_tiled32<WF, MODE, 6>(p, t, s);
-      default: return launch_tiled32<WF, MODE, 7>(p, t, s);
+      case 2: return launch_height<WF, MODE, 2>(p, t, s);
+      case 3: return launch_height<WF, MODE, 3>(p, t, s);
+      case 4: return launch_height<WF, MODE, 4>(p, t, s);
+      case 5: return launch_height<WF, MODE, 5>(p, t, s);
+      case 6: return launch_height<WF, MODE, 6>(p, t, s);
+      default: return launch_height<WF, MODE, 7>(p, t, s);
     }
   }
 }
