@@ -120,7 +120,12 @@ def ptr(t):
 
 
 def stream_handle(stream=None):
+    return ctypes.c_void_p(raw_stream() if stream is None else stream.cuda_stream)
+
+
+def raw_stream(index=None):
+    """The handle of a device's current stream (the current device's by default), without the Stream
+    object that torch.cuda.current_stream builds: 0.3 against 3 us a call."""
     import torch
 
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)

@@ -179,7 +179,8 @@ int forward_impl(const char* fn, const void* x, const void* wg, const void* wu, 
   // where the kernels take one (block-float weights, M > 32).  Fused into the split kernel's
   // staging, where every workgroup read every token row, it cost more than the pass and its
   // launch: gate/up 45 against 35 us at 1 and 16 tokens, 56 against 41 us at 32 (27B, bfp8).
-  const bool gemv = gemv_supported(M, H, I, di.num_cus);
+  GemvPlan pg, pd;
+  const bool gemv = plan_forward_gemv(M, H, I, di.num_cus, &pg, &pd);
   const bool stream_k = !gemv && stream_supported(M, H, I, di.num_cus);
   if (normw && (gemv || stream_k || fmt == QMLP_FMT_BF16)) {
     uint8_t* xn = (uint8_t*)ws + L.xn;
@@ -187,7 +188,7 @@ int forward_impl(const char* fn, const void* x, const void* wg, const void* wu, 
     a.x = xn;
     a.normw = nullptr;
   }
-  if (gemv) return launch_forward_gemv(a, di.num_cus, (hipStream_t)stream);
+  if (gemv) return launch_forward_gemv(a, pg, pd, (hipStream_t)stream);
   if (stream_k) return launch_forward_stream(a, di.num_cus, (hipStream_t)stream);
   if (tiled_supported(M, H, I)) return launch_forward_tiled(a, di.num_cus, (hipStream_t)stream);
   return set_error(QMLP_E_SHAPE, "%s: no kernel for M=%d H=%d I=%d", fn, M, H, I);

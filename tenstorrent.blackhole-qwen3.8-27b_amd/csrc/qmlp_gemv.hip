@@ -171,24 +171,11 @@ __device__ __forceinline__ void stage_b_finish(const GvParams& p, int kq, const 
         const u16x2 sub = __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, r & 0x7fff7fffu), d2);
         o[i] = __builtin_bit_cast(uint32_t, (u16x2)(sub << (u16x2){3, 3})) | (r & 0x80008000u);
       }
+      // The word arithmetic has no infinities or NaN: a row slice that holds one carries a NaN in its
+      // first word, which makes every output of the row not finite.  (Staging such a slice again
+      // in a branch of its own cost 0.4 us of a 56 us layer.)
+      if (c == 0 && tl == 0 && mb >= 0x7f80u) o[0] = 0x7e007e00u;
       *(u32x4*)(ldsb + lds_off((tl + c * TPR) * 8)) = u32x4{o[0], o[1], o[2], o[3]};
-    }
-  }
-  // The word arithmetic above has no infinities or NaN: a row slice that holds one is staged again
-  // with them (rare, decided once per row).
-  if (mb >= 0x7f80u) {
-    auto half = [](uint32_t b) {  // finite values: any, the row's products are not finite anyway
-      const uint32_t m = b & 0x7fffu;
-      return m < 0x7f80u ? 0x3c00u : (m == 0x7f80u ? 0x7c00u | (b & 0x8000u) : 0x7e00u);
-    };
-#pragma unroll
-    for (int c = 0; c < MAXCH; ++c) {
-      if (c < nch) {
-        uint32_t o[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = half(bs.v[c][i] & 0xffffu) | (half(bs.v[c][i] >> 16) << 16);
-        *(u32x4*)(ldsb + lds_off((tl + c * TPR) * 8)) = u32x4{o[0], o[1], o[2], o[3]};
-      }
     }
   }
 }
@@ -828,19 +815,15 @@ size_t gemv_part_bytes(int rows, int K, int nmat, int mg) {
 
 int gemv_groups(int M) { return M > 16 ? 2 : 1; }
 
-bool gemv_supported(int M, int H, int I, int num_cus) {
+bool plan_forward_gemv(int M, int H, int I, int num_cus, GemvPlan* gate_up, GemvPlan* down) {
   if (M < 1 || M > 32) return false;
   const int mg = gemv_groups(M);
-  GemvPlan a, b;
-  return plan_gemv(I, H, 2, mg, num_cus, &a) == 0 && plan_gemv(H, I, 1, mg, num_cus, &b) == 0;
+  return plan_gemv(I, H, 2, mg, num_cus, gate_up) == 0 && plan_gemv(H, I, 1, mg, num_cus, down) == 0;
 }
 
-int launch_forward_gemv(const ForwardArgs& a, int num_cus, hipStream_t s) {
+int launch_forward_gemv(const ForwardArgs& a, const GemvPlan& pg, const GemvPlan& pd, hipStream_t s) {
   const WsLayout L = ws_layout(a.M, a.H, a.I, a.fmt);
   const int fmt = a.fmt, mg = gemv_groups(a.M);
-  GemvPlan pg, pd;
-  if (plan_gemv(a.I, a.H, 2, mg, num_cus, &pg) || plan_gemv(a.H, a.I, 1, mg, num_cus, &pd))
-    return set_error(-1, "no weight-streaming split for M=%d H=%d I=%d", a.M, a.H, a.I);
   int* th = (int*)(a.ws + L.th);
   uint16_t* h = (uint16_t*)(a.ws + L.h);
   GvParams g{};

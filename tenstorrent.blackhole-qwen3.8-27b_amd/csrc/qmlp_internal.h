@@ -69,7 +69,8 @@ constexpr int kMaxSplit = 16;
 // mg: groups of 16 tokens (1 for M <= 16, 2 for M <= 32).
 int plan_gemv(int rows, int K, int nmat, int mg, int num_cus, GemvPlan* out);
 int gemv_groups(int M);
-bool gemv_supported(int M, int H, int I, int num_cus);
+// The plans of both projections, or false where no split fits.
+bool plan_forward_gemv(int M, int H, int I, int num_cus, GemvPlan* gate_up, GemvPlan* down);
 // Largest partial-slot buffer any device could need for this projection (workspace size).
 size_t gemv_part_bytes(int rows, int K, int nmat, int mg);
 
@@ -115,7 +116,7 @@ bool tiled_supported(int M, int H, int I);
 constexpr int kSplitMaxSlots = 256;
 size_t tiled_split_bytes(int M);
 void plan_tiles_info(int M, int H, int I, int fmt, bool down, int num_cus, int* out8);
-int launch_forward_gemv(const ForwardArgs& a, int num_cus, hipStream_t s);
+int launch_forward_gemv(const ForwardArgs& a, const GemvPlan& pg, const GemvPlan& pd, hipStream_t s);
 // Stream-K weight-streaming kernels for M <= 32 (qmlp_stream.hip).
 int plan_stream(int rows, int K, int num_cus, int* P, int* maxseg);
 bool stream_supported(int M, int H, int I, int num_cus);

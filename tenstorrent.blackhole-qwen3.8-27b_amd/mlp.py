@@ -259,9 +259,10 @@ class WorkspacePool:
 
     @staticmethod
     def _key(device, stream):
-        s = stream if stream is not None else torch.cuda.current_stream(device)
-        return (torch.device(device).index if torch.device(device).index is not None else torch.cuda.current_device(),
-                s.cuda_stream)
+        if not isinstance(device, torch.device):
+            device = torch.device(device)
+        index = device.index if device.index is not None else torch.cuda.current_device()
+        return index, (_lib.raw_stream(index) if stream is None else stream.cuda_stream)
 
     def reserve(self, nbytes, device, stream=None):
         """The workspace of (device, stream), grown to at least ``nbytes`` (outside capture only)."""
@@ -350,7 +351,7 @@ def load_mlp_weights(device, state_dict, tensor_cache_path=None, args=None, weig
     if device.type != "cuda":
         raise ValueError(f"device must be a GPU, got {device}")
     names = {"w1": "gate_proj", "w2": "down_proj", "w3": "up_proj"}
-    packed, pending = {}, []  # a matrix's conversion is checked while the next one's runs
+    packed, pending = {}, []  # conversions are checked once all are queued: a check waits for the stream
     for field, name in names.items():
         mfmt = down_fmt if field == "w2" else gu_fmt
         cache = None
@@ -382,10 +383,8 @@ def load_mlp_weights(device, state_dict, tensor_cache_path=None, args=None, weig
         packed[field] = _pack_weight_begin(w, mfmt, None)
         del w
         pending.append((packed[field], cache))
-        if len(pending) > 1:
-            _finish_load(*pending.pop(0), strict)
-    while pending:
-        _finish_load(*pending.pop(0), strict)
+    for pw, cache in pending:
+        _finish_load(pw, cache, strict)
     weights = MLPWeights(**packed)
     I, H = weights.w1.rows, weights.w1.cols
     if (weights.w3.rows, weights.w3.cols) != (I, H) or (weights.w2.rows, weights.w2.cols) != (H, I):
@@ -501,6 +500,7 @@ class Qwen36MLP:
         self.max_tokens = int(max_tokens)
         self.pool = workspace_pool if pool is None else pool
         nbytes = self._workspace_bytes(self.max_tokens)
+        self._ws_size = (self.max_tokens, nbytes)
         self.pool.reserve(nbytes, self.device)
         # torch.cuda.graph(g) without a stream captures on its own side stream: give it a workspace
         # too, so that the usual warm-up-then-capture pattern needs no stream argument
@@ -519,7 +519,11 @@ class Qwen36MLP:
         # sizes never shrink as M grows, so the reservation for max_tokens covers every smaller call
         if M > self.max_tokens and not torch.cuda.is_current_stream_capturing():
             self.max_tokens = M
-        return self.pool.reserve(self._workspace_bytes(max(M, self.max_tokens)), self.device)
+        tokens = max(M, self.max_tokens)
+        size = self._ws_size  # (tokens, bytes), replaced as a whole: threads may share an instance
+        if size[0] != tokens:
+            size = self._ws_size = (tokens, self._workspace_bytes(tokens))
+        return self.pool.reserve(size[1], self.device)
 
     def forward(self, x, residual=None, out=None, out_dtype=None):
         if not isinstance(x, torch.Tensor) or x.dtype != torch.bfloat16:
@@ -529,7 +533,7 @@ class Qwen36MLP:
         if x.device.type != "cuda":
             raise ValueError("activation must be on the GPU")
         shape = x.shape
-        x2d = x.reshape(-1, shape[-1])
+        x2d = x if x.dim() == 2 else x.reshape(-1, shape[-1])
         if not x2d.is_contiguous():
             x2d = x2d.contiguous()
         M = x2d.shape[0]
@@ -539,7 +543,7 @@ class Qwen36MLP:
         if residual is not None:
             if tuple(residual.shape) != tuple(shape):
                 raise ValueError("residual must have the activation's shape")
-            r2d = residual.reshape(M, shape[-1])
+            r2d = residual if residual.dim() == 2 else residual.reshape(M, shape[-1])
         o2d = None
         if out is not None:
             if tuple(out.shape) != tuple(shape):
@@ -549,7 +553,9 @@ class Qwen36MLP:
             o2d = out.reshape(M, shape[-1])
         y = mlp_forward(x2d, self.weights, residual=r2d, out=o2d, workspace=self._workspace_for(M),
                         out_dtype=out_dtype)
-        return y.reshape(shape) if out is None else out
+        if out is not None:
+            return out
+        return y if len(shape) == 2 else y.reshape(shape)
 
     __call__ = forward
 
@@ -562,7 +568,7 @@ class Qwen36MLP:
         if h.dim() < 1 or h.shape[-1] != self.weights.hidden:
             raise ValueError(f"h must end in hidden size {self.weights.hidden}, got {tuple(h.shape)}")
         shape = h.shape
-        h2d = h.reshape(-1, shape[-1])
+        h2d = h if h.dim() == 2 else h.reshape(-1, shape[-1])
         if not h2d.is_contiguous():
             h2d = h2d.contiguous()
         M = h2d.shape[0]
@@ -575,4 +581,6 @@ class Qwen36MLP:
             o2d = out.reshape(M, shape[-1])
         y = mlp_forward_rmsnorm(h2d, norm_weight, self.weights, eps=eps, out=o2d, workspace=self._workspace_for(M),
                                 out_dtype=out_dtype)
-        return y.reshape(shape) if out is None else out
+        if out is not None:
+            return out
+        return y if len(shape) == 2 else y.reshape(shape)
