@@ -593,9 +593,10 @@ __global__ __launch_bounds__(256) void sum_kernel(TlParams p, int mg) {
 
 // ---------------------------------------------------------------- host side
 
-// What a launch of tiled32_kernel costs, in us, as measured on MI355X: 21 token counts from 33 to
-// 2048 at the 27B shapes, every tile height and the splits within 1.4 x the best estimate, fitted to
-// 4 % rms with the points near the fastest weighted most.
+// What a launch of tiled32_kernel costs, in us, as measured on MI355X: 22 token counts from 33 to
+// 2048 at the 27B shapes (H = 5120, I = 17408), every tile height and the splits within 1.4 x the
+// best estimate, about 500 points per mode and format, fitted to 3-5 % rms with the points near the
+// fastest weighted most.  The plans chosen are 0.7 % slower on average than the fastest measured.
 struct TileCost {
   float step[8];   // one 64-K step of a tile of MG groups (0: height not built)
   float tile;      // a tile's, or a piece's, start and end
@@ -632,7 +633,7 @@ struct TilePlan {
 // split.  Before heights and multi-round splits were weighed against each other -- tiles of 64 or
 // 128 tokens, pieces within one round -- a count of tiles just above a round or a half round left
 // up to half the chip idle (27B layer, interleaved: 201 tokens bf4 205 us, now 166; 777 tokens bf16
-// 607, now 463).
+// 607, now 463; with sum_kernel 210 -> 159 and 614 -> 466).
 static void plan_mode(int mode, const TileCost& c, int M, int N, int C, int fmt, int slots, size_t part_bytes,
                       TilePlan* best) {
   const int nm = mode == kBoth ? 2 : 1, kst = C * kSteps;
