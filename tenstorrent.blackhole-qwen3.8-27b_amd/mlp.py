@@ -381,10 +381,11 @@ def load_mlp_weights(device, state_dict, tensor_cache_path=None, args=None, weig
             w = torch.as_tensor(w)
         w = w.to(device=device, dtype=torch.bfloat16).contiguous()
         packed[field] = _pack_weight_begin(w, mfmt, None)
+        pending.append((packed[field], cache, w))  # w: its memory may belong to another stream
         del w
-        pending.append((packed[field], cache))
-    for pw, cache in pending:
-        _finish_load(pw, cache, strict)
+    while pending:
+        pw, cache, w = pending.pop(0)
+        _finish_load(pw, cache, strict)  # the conversion has read w
     weights = MLPWeights(**packed)
     I, H = weights.w1.rows, weights.w1.cols
     if (weights.w3.rows, weights.w3.cols) != (I, H) or (weights.w2.rows, weights.w2.cols) != (H, I):

@@ -1,0 +1,58 @@
+"""Loading a layer without a GPU: what ``load_mlp_weights`` does around its conversions, with the
+conversion and its check replaced by stand-ins."""
+import weakref
+
+import pytest
+import torch
+
+I, H = 512, 256
+
+
+class _Source(torch.Tensor):
+    """A checkpoint tensor whose device copy is a tensor of this process, kept in ``copies`` weakly."""
+
+    copies = []
+
+    def to(self, *args, **kwargs):
+        t = torch.zeros(tuple(self.shape), dtype=torch.bfloat16)
+        _Source.copies.append(weakref.ref(t))
+        return t
+
+
+class _Checkpoint(dict):
+    """Makes a tensor at each access and keeps none, like a lazily read checkpoint."""
+
+    def __getitem__(self, name):
+        return torch.zeros(super().__getitem__(name)).as_subclass(_Source)
+
+
+def _checkpoint():
+    return _Checkpoint({"gate_proj.weight": (I, H), "up_proj.weight": (I, H), "down_proj.weight": (H, I)})
+
+
+@pytest.fixture
+def stand_ins(pkg, monkeypatch):
+    from qwen_mlp_amd import mlp
+
+    def begin(w, fmt, stream):
+        return mlp.PackedWeight(torch.zeros(0, dtype=torch.uint8), *w.shape, fmt)
+
+    monkeypatch.setattr(_Source, "copies", [])
+    monkeypatch.setattr(mlp, "_pack_weight_begin", begin)
+    monkeypatch.setattr(mlp, "_pack_weight_end", lambda pw, strict, stream: pw)
+    return mlp
+
+
+def test_sources_outlive_their_conversions(stand_ins, monkeypatch):
+    """A matrix's bf16 source lives until the check that waits for its conversion: dropped before,
+    memory that belongs to another stream could be handed out again while the conversion reads it."""
+    mlp = stand_ins
+    alive = []
+
+    def end(pw, strict, stream):
+        alive.append(_Source.copies[len(alive)]() is not None)
+        return pw
+
+    monkeypatch.setattr(mlp, "_pack_weight_end", end)
+    mlp.load_mlp_weights("cuda", _checkpoint())
+    assert alive == [True, True, True]
