@@ -352,40 +352,42 @@ def load_mlp_weights(device, state_dict, tensor_cache_path=None, args=None, weig
         raise ValueError(f"device must be a GPU, got {device}")
     names = {"w1": "gate_proj", "w2": "down_proj", "w3": "up_proj"}
     packed, pending = {}, []  # conversions are checked once all are queued: a check waits for the stream
-    for field, name in names.items():
-        mfmt = down_fmt if field == "w2" else gu_fmt
-        cache = None
-        if tensor_cache_path is not None:
-            from . import weight_cache
+    try:
+        for field, name in names.items():
+            mfmt = down_fmt if field == "w2" else gu_fmt
+            cache = None
+            if tensor_cache_path is not None:
+                from . import weight_cache
 
-            cache = weight_cache.cache_file(tensor_cache_path, name, mfmt)
-            pw = weight_cache.load(cache, device) if os.path.exists(cache) else None
-            if pw is not None:
-                if pw.fmt != mfmt:
-                    raise ValueError(f"cache entry {cache} holds {pw.fmt}, expected {mfmt}")
-                src = state_dict.get(f"{name}.weight") if hasattr(state_dict, "get") else None
-                if src is not None and tuple(src.shape) != (pw.rows, pw.cols):
-                    raise ValueError(f"cache entry {cache} is [{pw.rows}, {pw.cols}] but {name}.weight is "
-                                     f"{list(src.shape)}: stale cache")
-                header = (pw.max_row_norm, pw.flushed_groups)
-                _read_info(pw)  # the trailer the kernels read, not the file header's copy of it
-                if header != (pw.max_row_norm, pw.flushed_groups):
-                    raise ValueError(f"cache entry {cache}: header and packed trailer disagree")
-                if strict and pw.flushed_groups:
-                    raise ValueError(f"cache entry {cache}: {pw.flushed_groups} {mfmt} groups lie more than 19 "
-                                     "binades below their row maximum")
-                packed[field] = pw
-                continue
-        w = state_dict[f"{name}.weight"]
-        if not isinstance(w, torch.Tensor):
-            w = torch.as_tensor(w)
-        w = w.to(device=device, dtype=torch.bfloat16).contiguous()
-        packed[field] = _pack_weight_begin(w, mfmt, None)
-        pending.append((packed[field], cache, w))  # w: its memory may belong to another stream
-        del w
-    while pending:
-        pw, cache, w = pending.pop(0)
-        _finish_load(pw, cache, strict)  # the conversion has read w
+                cache = weight_cache.cache_file(tensor_cache_path, name, mfmt)
+                pw = weight_cache.load(cache, device) if os.path.exists(cache) else None
+                if pw is not None:
+                    if pw.fmt != mfmt:
+                        raise ValueError(f"cache entry {cache} holds {pw.fmt}, expected {mfmt}")
+                    src = state_dict.get(f"{name}.weight") if hasattr(state_dict, "get") else None
+                    if src is not None and tuple(src.shape) != (pw.rows, pw.cols):
+                        raise ValueError(f"cache entry {cache} is [{pw.rows}, {pw.cols}] but {name}.weight is "
+                                         f"{list(src.shape)}: stale cache")
+                    header = (pw.max_row_norm, pw.flushed_groups)
+                    _read_info(pw)  # the trailer the kernels read, not the file header's copy of it
+                    if header != (pw.max_row_norm, pw.flushed_groups):
+                        raise ValueError(f"cache entry {cache}: header and packed trailer disagree")
+                    if strict and pw.flushed_groups:
+                        raise ValueError(f"cache entry {cache}: {pw.flushed_groups} {mfmt} groups lie more than 19 "
+                                         "binades below their row maximum")
+                    packed[field] = pw
+                    continue
+            w = state_dict[f"{name}.weight"]
+            if not isinstance(w, torch.Tensor):
+                w = torch.as_tensor(w)
+            w = w.to(device=device, dtype=torch.bfloat16).contiguous()
+            packed[field] = _pack_weight_begin(w, mfmt, None)
+            pending.append((packed[field], cache, w))  # w: its memory may belong to another stream
+            del w
+    finally:  # also where a later matrix fails: those before it are checked and cached, their error first
+        while pending:
+            pw, cache, w = pending.pop(0)
+            _finish_load(pw, cache, strict)  # the conversion has read w
     weights = MLPWeights(**packed)
     I, H = weights.w1.rows, weights.w1.cols
     if (weights.w3.rows, weights.w3.cols) != (I, H) or (weights.w2.rows, weights.w2.cols) != (H, I):

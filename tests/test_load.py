@@ -56,3 +56,25 @@ def test_sources_outlive_their_conversions(stand_ins, monkeypatch):
     monkeypatch.setattr(mlp, "_pack_weight_end", end)
     mlp.load_mlp_weights("cuda", _checkpoint())
     assert alive == [True, True, True]
+
+
+def test_a_later_failure_keeps_what_came_before(stand_ins, monkeypatch, tmp_path):
+    """Matrices load in the order gate, down, up: where a later one is missing, those before it
+    have been checked and cached, and where one of those is refused, that is the error."""
+    mlp = stand_ins
+    from qwen_mlp_amd import weight_cache
+
+    saved = []
+    monkeypatch.setattr(weight_cache, "save", lambda path, pw: saved.append((pw.rows, pw.cols)))
+    sd = _checkpoint()
+    del sd["up_proj.weight"]
+    with pytest.raises(KeyError, match="up_proj"):
+        mlp.load_mlp_weights("cuda", sd, tensor_cache_path=str(tmp_path))
+    assert saved == [(I, H), (H, I)]
+
+    def end(pw, strict, stream):
+        raise ValueError("non-finite")
+
+    monkeypatch.setattr(mlp, "_pack_weight_end", end)
+    with pytest.raises(ValueError, match="non-finite"):
+        mlp.load_mlp_weights("cuda", sd, tensor_cache_path=str(tmp_path))
