@@ -261,6 +261,8 @@ class WorkspacePool:
     def _key(device, stream):
         if not isinstance(device, torch.device):
             device = torch.device(device)
+        if device.type != "cuda":
+            raise ValueError(f"a workspace needs a GPU, got {device}")
         index = device.index if device.index is not None else torch.cuda.current_device()
         return index, (_lib.raw_stream(index) if stream is None else stream.cuda_stream)
 

@@ -78,3 +78,16 @@ def test_a_later_failure_keeps_what_came_before(stand_ins, monkeypatch, tmp_path
     monkeypatch.setattr(mlp, "_pack_weight_end", end)
     with pytest.raises(ValueError, match="non-finite"):
         mlp.load_mlp_weights("cuda", sd, tensor_cache_path=str(tmp_path))
+
+
+def test_pool_refuses_a_device_that_is_not_a_gpu(pkg, monkeypatch):
+    """Also where the current GPU's stream already holds a workspace."""
+    from qwen_mlp_amd import _lib
+
+    pool = pkg.WorkspacePool()
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(_lib, "raw_stream", lambda index=None: 0)
+    pool._ws[pool._key("cuda", None)] = torch.zeros(64, dtype=torch.uint8)
+    assert pool.reserve(64, "cuda:0").numel() == 64
+    with pytest.raises(ValueError, match="cpu"):
+        pool.reserve(64, "cpu")
