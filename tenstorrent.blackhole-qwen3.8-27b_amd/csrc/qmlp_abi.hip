@@ -171,7 +171,7 @@ int forward_impl(const char* fn, const void* x, const void* wg, const void* wu, 
   DeviceInfo di;
   if (int rc = current_device_info(&di)) return rc;
   ForwardArgs a{x, (const uint8_t*)wg, (const uint8_t*)wu, (const uint8_t*)wd, residual, out, (uint8_t*)ws,
-                M, H, I, fmt, (flags & QMLP_OUT_F32) ? 1 : 0, (flags & QMLP_RESIDUAL_F32) ? 1 : 0, normw, eps};
+                M, H, I, fmt, (flags & QMLP_OUT_F32) ? 1 : 0, (flags & QMLP_RESIDUAL_F32) ? 1 : 0, normw, eps, false};
   // M <= 32: split-K weight streaming with LDS-staged activations; where no such split fits (a K
   // too long for the staged activations, or a device too small for the split's registers),
   // M <= 32: stream-K weight streaming with activations read from L2; larger M: the LDS-tiled
@@ -187,6 +187,7 @@ int forward_impl(const char* fn, const void* x, const void* wg, const void* wu, 
     if (int rc = launch_rmsnorm(x, normw, eps, M, H, xn, (hipStream_t)stream)) return rc;
     a.x = xn;
     a.normw = nullptr;
+    a.normed = true;
   }
   if (gemv) return launch_forward_gemv(a, pg, pd, (hipStream_t)stream);
   if (stream_k) return launch_forward_stream(a, di.num_cus, (hipStream_t)stream);

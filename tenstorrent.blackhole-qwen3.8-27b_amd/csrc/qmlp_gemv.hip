@@ -67,6 +67,7 @@ constexpr int kPssStride = 64;  // floats of token sums per workgroup
 
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 // Per-(matrices, token groups) constants.  Both bound the registers of one wave to ~48 VGPRs:
 //   kMaxSeg: parked partial tiles per wave (the planner rejects splits that need more);
@@ -114,7 +115,11 @@ __device__ __forceinline__ void stage_b_issue(const GvParams& p, int k0, int kq,
   for (int c = 0; c < MAXCH; ++c) bs.v[c] = *(const u32x4*)(row + (tl + min(c, nch - 1) * TPR) * 8);
 }
 
-template <int NW, int MAXCH, int MG>
+// EXACT (rows behind the norm): every value as fp16(x * 2^t) rounded to nearest, subnormals included,
+// so that values down to about 2^-38 of the range's maximum count; without it those below 2^-28 are
+// lost.  v_cvt_pk_f16_f32 makes it as fast as the packed words: the 27B layer behind the norm takes
+// 57.8 us at 1 token (bfp8), 48.3 at 16 (bf4) and 68.7 at 32 (bfp8) with either.
+template <int NW, int MAXCH, int MG, bool EXACT>
 __device__ __forceinline__ void stage_b_finish(const GvParams& p, int kq, const BStage<MAXCH>& bs, uint8_t* ldsb,
                                                int* lds_t, float* lds_ss) {
   constexpr int TPR = NW * 64 / (16 * MG);
@@ -130,10 +135,11 @@ __device__ __forceinline__ void stage_b_finish(const GvParams& p, int kq, const 
       if (c < nch) *(u32x4*)(ldsb + lds_off((tl + c * TPR) * 8)) = bs.v[c];
     return;
   }
-  // bf16 x -> fp16 * 2^t on packed 16-bit words: the magnitudes' integer maximum is the
-  // maximum value, the sum of squares comes from v_dot2_f32_bf16, and the conversion is
+  // bf16 x -> fp16 * 2^t, the magnitudes' integer maximum being the maximum value.  Without EXACT on
+  // packed 16-bit words: the sum of squares comes from v_dot2_f32_bf16, and the conversion is
   // fp16 bits = ((|x| bits - ((112 - t) << 7)) << 3) | sign, exact while x * 2^t is a normal
-  // half; values below 2^-14 after scaling (2^-28 of the range maximum) are flushed to zero.
+  // half; smaller values (2^-28 of the range maximum) are lost: below 2^-15 after scaling they
+  // become zero, from there up to 2^-14 too small.
   u16x2 mx2 = {0, 0};
   float ss = 0.f;
 #pragma unroll
@@ -143,7 +149,12 @@ __device__ __forceinline__ void stage_b_finish(const GvParams& p, int kq, const 
       for (int i = 0; i < 4; ++i) {
         const uint32_t r = bs.v[c][i];
         mx2 = __builtin_elementwise_max(mx2, __builtin_bit_cast(u16x2, r & 0x7fff7fffu));
-        ss = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, r), __builtin_bit_cast(bf16x2, r), ss, false);
+        if constexpr (EXACT) {
+          const float lo = __uint_as_float(r << 16), hi = __uint_as_float(r & 0xffff0000u);
+          ss = fmaf(hi, hi, fmaf(lo, lo, ss));
+        } else {
+          ss = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, r), __builtin_bit_cast(bf16x2, r), ss, false);
+        }
       }
   uint32_t mb = max((uint32_t)mx2.x, (uint32_t)mx2.y);
 #pragma unroll
@@ -154,10 +165,27 @@ __device__ __forceinline__ void stage_b_finish(const GvParams& p, int kq, const 
   const float mxf = bf16_to_f32((uint16_t)mb);
   int e2 = 0;
   if (mxf > 0.f) frexpf(mxf, &e2);
-  const int t = mxf > 0.f ? min(15 - e2, 112) : 0;
+  const int t = mxf > 0.f ? (EXACT ? 15 - e2 : min(15 - e2, 112)) : 0;
   if (tl == 0) {
     lds_t[m] = t;
     lds_ss[m] = ss;
+  }
+  if constexpr (EXACT) {
+#pragma unroll
+    for (int c = 0; c < MAXCH; ++c) {
+      if (c < nch) {
+        uint32_t o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t r = bs.v[c][i];
+          const f32x2 x = {__builtin_amdgcn_ldexpf(__uint_as_float(r << 16), t),
+                           __builtin_amdgcn_ldexpf(__uint_as_float(r & 0xffff0000u), t)};
+          o[i] = as_u32(__builtin_convertvector(x, f16x2));
+        }
+        *(u32x4*)(ldsb + lds_off((tl + c * TPR) * 8)) = u32x4{o[0], o[1], o[2], o[3]};
+      }
+    }
+    return;
   }
   const uint32_t dd = (uint32_t)(112 - t) << 7;
   const u16x2 d2 = __builtin_bit_cast(u16x2, dd | (dd << 16));
@@ -359,7 +387,7 @@ __device__ __forceinline__ void gepilogue(const GvParams& p, int t, const f32x4 
 
 // ---------------------------------------------------------------- kernel
 
-template <int WF, int NMAT, int NW, int MAXCH, int MG>
+template <int WF, int NMAT, int NW, int MAXCH, int MG, bool EXACT>
 __global__ __launch_bounds__(NW * 64) void gemv_kernel(GvParams p) {
   constexpr int SPS = WF ? 4 : 2;  // K-steps per register stage
   constexpr int SPU = kSteps / SPS;
@@ -411,7 +439,7 @@ __global__ __launch_bounds__(NW * 64) void gemv_kernel(GvParams p) {
   stage_b_issue<NW, MAXCH, MG>(p, c0 * kSuperK, kq, bs);
   gload(s0, p, blk_base, P0, lw, le);
   gload(s1, p, blk_base, P1, lw, le);  // repeats stage 0 when nst == 1
-  stage_b_finish<NW, MAXCH, MG>(p, kq, bs, ldsb, s_t, s_ss);
+  stage_b_finish<NW, MAXCH, MG, EXACT>(p, kq, bs, ldsb, s_t, s_ss);
   gload(s2, p, blk_base, P2, lw, le);
   __syncthreads();
 
@@ -773,9 +801,9 @@ static int enable_large_lds(const void* kern, const char* what) {
   return 0;
 }
 
-template <int WF, int NMAT, int MAXCH, int MG>
+template <int WF, int NMAT, int MAXCH, int MG, bool EXACT>
 static int launch_gemv_ch(const GvParams& p, size_t lds, hipStream_t s) {
-  auto kern = gemv_kernel<WF, NMAT, kGemvNW, MAXCH, MG>;
+  auto kern = gemv_kernel<WF, NMAT, kGemvNW, MAXCH, MG, EXACT>;
   if (int rc = enable_large_lds((const void*)kern, "gemv_kernel")) return rc;
   launch_timed(NMAT == 2 ? 0 : 1, kern, dim3(p.P), dim3(kGemvNW * 64), lds, s, p);
   return check_launch("gemv_kernel");
@@ -783,17 +811,17 @@ static int launch_gemv_ch(const GvParams& p, size_t lds, hipStream_t s) {
 
 // The staging register array is sized by a small set of buckets (loads beyond KQ * MG are clamped
 // duplicates).
-template <int WF, int NMAT, int MG>
+template <int WF, int NMAT, int MG, bool EXACT>
 static int launch_gemv_mg(const GvParams& p, size_t lds, hipStream_t s) {
   const int nch = p.KQ * MG;
-  if (nch <= 4) return launch_gemv_ch<WF, NMAT, 4, MG>(p, lds, s);
-  if (nch <= 10) return launch_gemv_ch<WF, NMAT, 10, MG>(p, lds, s);
-  return launch_gemv_ch<WF, NMAT, kGemvMaxChunks, MG>(p, lds, s);
+  if (nch <= 4) return launch_gemv_ch<WF, NMAT, 4, MG, EXACT>(p, lds, s);
+  if (nch <= 10) return launch_gemv_ch<WF, NMAT, 10, MG, EXACT>(p, lds, s);
+  return launch_gemv_ch<WF, NMAT, kGemvMaxChunks, MG, EXACT>(p, lds, s);
 }
 
-template <int WF, int NMAT>
+template <int WF, int NMAT, bool EXACT = false>
 static int launch_gemv(const GvParams& p, int mg, size_t lds, hipStream_t s) {
-  return mg == 2 ? launch_gemv_mg<WF, NMAT, 2>(p, lds, s) : launch_gemv_mg<WF, NMAT, 1>(p, lds, s);
+  return mg == 2 ? launch_gemv_mg<WF, NMAT, 2, EXACT>(p, lds, s) : launch_gemv_mg<WF, NMAT, 1, EXACT>(p, lds, s);
 }
 
 size_t gemv_part_bytes(int rows, int K, int nmat, int mg) {
@@ -852,9 +880,9 @@ int launch_forward_gemv(const ForwardArgs& a, const GemvPlan& pg, const GemvPlan
   g.pss = (float*)(a.ws + L.pss);
   g.counters = (int*)(a.ws + L.counters_gu);
   const size_t lg = gemv_lds_bytes(pg, 2, mg);
-  int rc = fmt == 2   ? launch_gemv<2, 2>(g, mg, lg, s)
-           : fmt == 1 ? launch_gemv<1, 2>(g, mg, lg, s)
-                      : launch_gemv<0, 2>(g, mg, lg, s);
+  int rc = fmt == 0   ? launch_gemv<0, 2>(g, mg, lg, s)
+           : fmt == 1 ? (a.normed ? launch_gemv<1, 2, true>(g, mg, lg, s) : launch_gemv<1, 2>(g, mg, lg, s))
+                      : (a.normed ? launch_gemv<2, 2, true>(g, mg, lg, s) : launch_gemv<2, 2>(g, mg, lg, s));
   if (rc) return rc;
   GvParams d{};
   d.w0 = a.wd;

@@ -104,6 +104,7 @@ struct ForwardArgs {
   int out_f32, res_f32;  // fp32 output / fp32 residual instead of bf16
   const void* normw;     // RMSNorm prologue: bf16 [H] weight (gain 1 + w), or null
   float eps;
+  bool normed;           // x holds rows that the RMSNorm pass wrote
 };
 // bfp8: x -> x16 = fp16(x * 2^tx[m]) and the h scale th[m], for all M tokens (qmlp_prep.hip).
 int launch_prep(const ForwardArgs& a, hipStream_t s);

@@ -64,6 +64,49 @@ def test_non_finite_rows_stay_in_their_rows(pkg, cuda, fmt, M):
         assert not torch.isfinite(got[[2, 4]]).any()
 
 
+@pytest.mark.parametrize("fmt", ["bfp8", "bf4"])
+@pytest.mark.parametrize("H", [2048, 8448])
+@pytest.mark.parametrize("M", [1, 16, 24])
+@pytest.mark.parametrize("depth", [29, 31, 34])
+def test_normalised_rows_keep_small_values(pkg, cuda, fmt, H, M, depth):
+    """Behind the norm, values far below their K range's maximum still count: one channel of each
+    256 is 2^depth times larger than the others, gate reads only those channels and up only the
+    others.  As fp16 with the maximum in [2^14, 2^15) the others are subnormal (6 bits of them left
+    at depth 34; each is rounded on its own, and up sums thousands); the product stays near
+    2^(depth - 27) times below the h bound, 11 bits or a few less."""
+    import numpy as np
+    import torch
+    from oracle import bf16 as obf16
+
+    I = 512
+    g = torch.Generator(cuda).manual_seed(H + M + depth)
+
+    def mantissas(*shape):
+        return 1.0 + torch.rand(shape, generator=g, device=cuda)
+
+    big = torch.arange(0, H, 256, device=cuda)
+    group = torch.zeros(H, dtype=torch.bool, device=cuda)
+    group[(big[:, None] + torch.arange(16, device=cuda)).flatten()] = True
+    gate = torch.zeros(I, H, device=cuda)
+    gate[:, big] = 0.125
+    up = mantissas(I, H) * 0.25
+    up[:, group] = 0.0
+    sd = {"gate_proj.weight": gate.bfloat16(), "up_proj.weight": up.bfloat16(),
+          "down_proj.weight": torch.randn(H, I, generator=g, device=cuda).bfloat16()}
+    x = mantissas(M, H) * 2.0 ** -depth
+    x[:, big] = mantissas(M, 1).expand(M, big.numel())
+    x = x.bfloat16()
+    mlp = pkg.Qwen36MLP(cuda, sd, weight_format=fmt, max_tokens=M)
+    y = mlp.forward_rmsnorm(x, torch.zeros(H, dtype=torch.bfloat16, device=cuda), eps=1e-6, out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    hw = host_weights(pkg, sd, fmt)
+    xf = x.float().cpu().numpy()
+    n = obf16.round_f32(omlp.rmsnorm(xf, np.zeros(H, np.float32), 1e-6))
+    ref = omlp.swiglu(n, hw["gate_proj"], hw["up_proj"], hw["down_proj"], dtype=np.float64)
+    small = ~group.cpu().numpy()  # where the residual is too small to round the sum
+    check(y.cpu().numpy()[:, small] - xf[:, small], ref[:, small], f"small values {fmt} H={H} M={M} 2^-{depth}")
+
+
 @pytest.mark.parametrize("fmt", ["bf16", "bfp8", "bf4"])
 @pytest.mark.parametrize("rows,cols", [(16, 256), (48, 2048), (16, 2304), (32, 4352), (16, 45056), (16, 45312)])
 def test_quantize_pack_matches_the_separate_passes(pkg, cuda, fmt, rows, cols):
