@@ -615,7 +615,14 @@ __global__ __launch_bounds__(256) void sum_kernel(TlParams p, int mg) {
 // What a launch of tiled32_kernel costs, in us, as measured on MI355X: 22 token counts from 33 to
 // 2048 at the 27B shapes (H = 5120, I = 17408), every tile height and the splits within 1.4 x the
 // best estimate, about 500 points per mode and format, fitted to 3-5 % rms with the points near the
-// fastest weighted most.  The plans chosen are 0.7 % slower on average than the fastest measured.
+// fastest weighted most.  The plans chosen are 0.7 % slower on average than the fastest measured there
+// (0.9-2.1 % in a later run on another box, at most 12 %, below 100 tokens).  At other shapes
+// (H = 1024-5120, I = 3072-16640, 48-2048 tokens) the estimates are up to a fifth too high, as tiles
+// over a short K overlap their ends, and the plans are 0.3 (bf4), 1.0 (bf16) and 1.3 % (bfp8) slower
+// than the fastest for gate/up, 1.2-1.7 and 3.5 % (bf16) for down, single ones by up to 24 %.
+// kCostPair16's publish was fitted as 0 at the 27B shapes; at 3072 x 8192 that split tiles which
+// whole ones beat, 58.9 against 45.3 us at 400 tokens and 44.1 against 34.0 at 259.  With .003 the
+// bf16 gate/up plans are 1.1 % slower than the fastest on average over all shapes, 2.1 % with 0.
 struct TileCost {
   float step[8];   // one 64-K step of a tile of MG groups (0: height not built)
   float tile;      // a tile's, or a piece's, start and end
@@ -628,7 +635,7 @@ struct TileCost {
 };
 constexpr TileCost kCostPair8{{0, 0, .53f, .75f, .92f, 1.15f, 1.33f, 1.55f}, 1.5f, 4.5f, 7.9f, .006f, .03f, 8.0f, .08f};
 constexpr TileCost kCostPair4{{0, 0, .48f, .65f, .89f, 1.20f, 1.30f, 1.51f}, 0.9f, 4.0f, 7.3f, .007f, .07f, 3.7f, .01f};
-constexpr TileCost kCostPair16{{0, 0, .57f, .78f, .92f, 1.13f, 1.26f, 1.46f}, 4.9f, 6.7f, 5.6f, .000f, .16f, 6.3f, .10f};
+constexpr TileCost kCostPair16{{0, 0, .57f, .78f, .92f, 1.13f, 1.26f, 1.46f}, 4.9f, 6.7f, 5.6f, .003f, .16f, 6.3f, .10f};
 constexpr TileCost kCostBoth{{0, 0, 1.02f, 0, 1.60f, 0, 0, 0}, 3.2f, 0.0f, 7.3f, .009f, .04f, 3.1f, .09f};
 constexpr TileCost kCostDown8{{0, 0, .53f, .75f, .93f, 1.16f, 1.36f, 1.61f}, 3.1f, 3.9f, 5.7f, .005f, .08f, 4.7f, .00f};
 constexpr TileCost kCostDown16{{0, 0, .55f, .73f, .87f, 1.07f, 1.20f, 1.40f}, 5.9f, 6.1f, 7.9f, .006f, .05f, 6.0f, .09f};

@@ -234,6 +234,26 @@ def test_tile_plans_cover_the_outputs_and_fit(pkg, H, I, fmt):
         assert pkg.lib().qmlp_plan_tiles(*bad, 0, 256, out) != 0
 
 
+# us of bf16 gate/up launches on MI355X by plan: (token rows of a tile, pieces of a split tile).
+MEASURED_TILES = [
+    (1024, 13312, 2048, {(192, 2): 139.7, (192, 1): 132.8, (128, 1): 137.3}),
+    (1536, 6144, 1400, {(192, 2): 74.2, (160, 1): 61.5}),
+    (3072, 8192, 259, {(160, 2): 44.1, (96, 1): 34.0}),
+    (3072, 8192, 400, {(224, 2): 58.9, (128, 1): 45.3}),
+    (4096, 12288, 640, {(160, 2): 135.0, (128, 1): 119.1}),
+    (5120, 17408, 777, {(224, 8): 293.0, (160, 1): 292.7, (224, 6): 287.4}),
+]
+
+
+@pytest.mark.parametrize("H,I,M,us", MEASURED_TILES)
+def test_tile_plans_are_near_the_fastest_measured(pkg, H, I, M, us):
+    """Where tiles could run whole or split, the plan picked is within 5 % of the fastest measured
+    (runs of one plan differ by 1-2 %)."""
+    out = (ctypes.c_int * 8)()
+    assert pkg.lib().qmlp_plan_tiles(M, H, I, 0, 0, 256, out) == 0
+    assert us[out[1], out[4]] <= 1.05 * min(us.values()), list(out)
+
+
 def test_plan_split_rejects_bad_widths(pkg):
     out = (ctypes.c_int * 6)()
     assert pkg.lib().qmlp_plan_split(17408, 5120, 2, 0, 256, out) != 0
