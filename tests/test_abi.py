@@ -234,6 +234,33 @@ def test_tile_plans_cover_the_outputs_and_fit(pkg, H, I, fmt):
         assert pkg.lib().qmlp_plan_tiles(*bad, 0, 256, out) != 0
 
 
+def test_gpu_tile_shapes_reach_every_instance(pkg):
+    """The plans of TILE_SHAPES launch every tiled32_kernel and sum_kernel that the dispatch can
+    (launch_height, launch_mode): features and matrices of a tile, its height, and whether the one
+    token block's weights pass the L2 by."""
+    from test_gpu_kernel_edges import TILE_SHAPES
+
+    fmts, out, got = ("bf16", "bfp8", "bf4"), (ctypes.c_int * 8)(), set()
+    for (H, I, M), fmt in ((s, f) for s in TILE_SHAPES for f in fmts):
+        for down in (0, 1):
+            assert pkg.lib().qmlp_plan_tiles(M, H, I, fmts.index(fmt), down, 256, out) == 0
+            feats, toks, _, nfull, ks = list(out)[:5]
+            wf = "bfp8" if down and fmt == "bf4" else fmt
+            mode = "down" if down else ("pair" if feats == 128 else "both")
+            got.add((wf, mode, toks // 32, M <= toks and wf != "bf4" and toks <= 96))
+            if ks > 1:
+                got.add((wf, mode, "sum behind whole rounds" if nfull else "sum"))
+    want = set()
+    for wf, mode in (("bf16", "down"), ("bfp8", "down"), ("bf16", "pair"), ("bfp8", "pair"), ("bf4", "pair"),
+                     ("bfp8", "both"), ("bf4", "both")):
+        want |= {(wf, mode, "sum"), (wf, mode, "sum behind whole rounds")}
+        for mg in (2, 4) if mode == "both" else range(2, 8):
+            want.add((wf, mode, mg, False))
+            if wf != "bf4" and mg <= 3:
+                want.add((wf, mode, mg, True))
+    assert sorted(want - got, key=str) == []
+
+
 # us of bf16 gate/up launches on MI355X by plan: (token rows of a tile, pieces of a split tile).
 MEASURED_TILES = [
     (1024, 13312, 2048, {(192, 2): 139.7, (192, 1): 132.8, (128, 1): 137.3}),

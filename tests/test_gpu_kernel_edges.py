@@ -146,14 +146,21 @@ def test_quantize_pack_matches_the_separate_passes(pkg, cuda, fmt, rows, cols):
             mlp.pack_weight(w, fmt)
 
 
+# (H, I, M) whose plans, over the three formats, take every built tile: each height in each mode, with
+# one token block and with several, and each mode's sums (tests/test_abi.py checks that they do).
+TILE_SHAPES = ([(2048, 6144, M) for M in (33, 65, 97, 129, 161, 193, 225, 321, 385, 449, 577, 777, 1153)]
+               + [(5120, 17408, M) for M in (68, 97, 201, 321, 449, 705, 777, 1281)]
+               + [(5376, 12288, 300), (256, 2560, 100), (2560, 256, 640), (768, 2048, 1800), (256, 10240, 1800),
+                  (5120, 8192, 68), (768, 256, 33), (512, 3072, 33), (256, 17408, 68), (256, 5120, 2048),
+                  (5120, 256, 2048), (3072, 4096, 1400), (1536, 17408, 500), (5120, 8192, 1600)])
+
+
 @pytest.mark.parametrize("fmt", ["bf16", "bfp8", "bf4"])
-@pytest.mark.parametrize("H,I,M", [(2048, 6144, M) for M in (33, 65, 97, 129, 161, 193, 225, 321, 385, 449, 577, 777, 1153)]
-                         + [(5120, 17408, M) for M in (97, 201, 321, 449, 705, 777, 1281)]
-                         + [(5376, 12288, 300), (256, 2560, 100), (2560, 256, 640)])
+@pytest.mark.parametrize("H,I,M", TILE_SHAPES)
 def test_tile_heights_and_splits(pkg, cuda, fmt, H, I, M):
     """Many-token tiles of every height with one live token row in the last block or a ragged one,
-    whole, split from the first tile on, and split behind whole rounds (a plan for every M: the
-    printed line); plain and behind the norm, twice."""
+    whole, split from the first tile on, and split behind whole rounds (the printed line is the
+    plan); plain and behind the norm, twice."""
     import ctypes
 
     import numpy as np
