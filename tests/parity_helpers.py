@@ -26,6 +26,17 @@ def record_margin(what, kind, ratio):
         f.write(json.dumps({"test": test, "what": what, "kind": kind, "ratio": round(float(ratio), 4)}) + "\n")
 
 
+def assert_splits_behind_whole_rounds(pkg, fmt, H, I, M):
+    """Both projections of a call above 32 tokens run whole rounds of tiles and then tiles whose K
+    range is split, on 256 CUs: what a test of that path relies on."""
+    import ctypes
+
+    out = (ctypes.c_int * 8)()
+    for down in (0, 1):
+        assert pkg.lib().qmlp_plan_tiles(M, H, I, {"bf16": 0, "bfp8": 1, "bf4": 2}[fmt], down, 256, out) == 0
+        assert out[3] > 0 and out[4] > 1, f"{fmt} H={H} I={I} M={M} {'down' if down else 'gate/up'}: {list(out)}"
+
+
 def bits(t):
     import torch
 

@@ -22,7 +22,8 @@ import numpy as np
 import pytest
 
 from oracle import mlp as omlp
-from parity_helpers import check, check_bf16, check_fp16_h, check_rows, host_weights, oracle
+from parity_helpers import assert_splits_behind_whole_rounds, check, check_bf16, check_fp16_h, check_rows
+from parity_helpers import host_weights, oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -92,8 +93,8 @@ def test_rmsnorm_prologue_27b_m2048_sampled_rows(pkg, cuda):
 @pytest.mark.parametrize("M", [48, 64, 128, 160, 256])
 def test_midwidth_27b_sampled_rows(pkg, cuda, fmt, M):
     """The 27B layer at a few dozen to a few hundred tokens (long verify windows, short prefill
-    chunks): fewer tiles than CUs, so every tile splits its K range (gate/up 3-4 pieces, down up to
-    8; with bf16 weights the down projection only) and the pieces finish the tile together;
+    chunks): every down tile splits its K range and a second launch adds the pieces; gate/up tiles,
+    by count and format, run whole, split from the first on or split behind a whole round;
     checked on the sampled rows of every 64-token block, the bf16 output against the fp32 one
     rounded once."""
     import torch
@@ -288,8 +289,8 @@ def test_heavy_tailed_27b(pkg, cuda, fmt):
 
 
 def test_heavy_tailed_rmsnorm_prologue(pkg, cuda):
-    """The fused RMSNorm prologue (M <= 32) and its separate pass (M > 32) on heavy-tailed h: the
-    norm equalises the rows, so the global bar applies."""
+    """The RMSNorm pass before the M <= 32 kernel and with the fp16 conversion (M > 32) on heavy-tailed
+    h: the norm equalises the rows, so the global bar applies."""
     import torch
 
     H, I = 1024, 3072
@@ -338,13 +339,14 @@ def test_poisoned_outputs_and_guard_bands(pkg, cuda, fmt, M):
     _poisoned_case(pkg, cuda, fmt, M, 1024, 3072)
 
 
-@pytest.mark.parametrize("fmt", ["bfp8", "bf4"])
-@pytest.mark.parametrize("H,I", [(1024, 4352), (5376, 2048)])
+@pytest.mark.parametrize("fmt,H,I", [(f, H, I) for f in ("bfp8", "bf4") for H, I in ((1024, 4352), (5376, 2048))]
+                         + [(f, 4352, 10240) for f in ("bf16", "bfp8", "bf4")])
 def test_poisoned_split_pieces(pkg, cuda, fmt, H, I):
-    """The poisoned-buffer checks at 2048 tokens on shapes whose last tiles split their K range
-    (gate/up at I = 4352: 16 tiles in 4 pieces; down at H = 5376: 80 tiles in 3 pieces), so that
-    the pieces' partial tiles go through the NaN-filled workspace and their counters must come
-    back to zero."""
+    """The poisoned-buffer checks at 2048 tokens on shapes that split K, so that the pieces' partial
+    tiles go through the NaN-filled workspace: every down tile at I = 4352, the tiles behind whole
+    rounds in both projections at H = 4352, I = 10240; H = 5376 runs whole tiles only."""
+    if H == 4352:
+        assert_splits_behind_whole_rounds(pkg, fmt, H, I, 2048)
     _poisoned_case(pkg, cuda, fmt, 2048, H, I)
 
 
@@ -385,7 +387,7 @@ def _poisoned_case(pkg, cuda, fmt, M, H, I):
                 check(y, ref, f"poisoned {fmt} M={M} fp32 run {run}")
             else:
                 check_bf16(y, ref, f"poisoned {fmt} M={M} run {run}")
-    # the RMSNorm entry point (fused prologue at M <= 32, separate pass otherwise), in place
+    # the RMSNorm entry point, in place
     nw = (torch.randn(H, generator=torch.Generator(cuda).manual_seed(3), device=cuda) * 0.3).to(torch.bfloat16)
     ws_buf, ws = _guarded(nbytes, NAN_BYTE, cuda)
     ws[:_lib.WS_COUNTER_BYTES] = 0

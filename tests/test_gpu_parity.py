@@ -12,7 +12,8 @@ from oracle import mlp as omlp
 
 pytestmark = pytest.mark.gpu
 
-from parity_helpers import TOL, bits as _bits, check as _check, check_bf16 as _check_bf16  # noqa: E402
+from parity_helpers import TOL, assert_splits_behind_whole_rounds  # noqa: E402
+from parity_helpers import bits as _bits, check as _check, check_bf16 as _check_bf16  # noqa: E402
 from parity_helpers import host_weights as _host_weights, oracle as _oracle  # noqa: E402
 
 
@@ -290,16 +291,18 @@ def test_bitwise_deterministic(pkg, cuda, fmt):
 
 
 @pytest.mark.parametrize("fmt", ["bf16", "bfp8", "bf4"])
-@pytest.mark.parametrize("H,I,M", [(1024, 4352, 2048), (5376, 2048, 2048), (1024, 3072, 64)])
+@pytest.mark.parametrize("H,I,M", [(1024, 4352, 2048), (5376, 2048, 2048), (1024, 3072, 64), (4352, 10240, 2048)])
 def test_prefill_bitwise_deterministic(pkg, cuda, fmt, H, I, M):
     """Many-token forwards repeated give identical bits, also where tiles split their K range into
-    pieces whose partial tiles meet in the workspace and are added in a fixed order: at 2048
-    tokens the tiles beyond the last whole round (gate/up at I = 4352: 16 tiles in 4 pieces; down
-    at H = 5376: 80 tiles in 3 pieces), at 64 tokens every tile."""
+    pieces whose partial tiles are added in a fixed order: I = 10240, in both projections, behind whole
+    rounds; I = 3072 and I = 4352, every down tile (and with block-float weights every gate/up tile
+    at 64 tokens); H = 5376 is whole tiles only."""
     import torch
     from qwen_mlp_amd import workloads
 
     print(f"case prefill determinism {fmt} H={H} I={I} M={M}", flush=True)
+    if H == 4352:
+        assert_splits_behind_whole_rounds(pkg, fmt, H, I, M)
     sd = workloads.state_dict(H, I, layer=5, device=cuda)
     mlp = pkg.Qwen36MLP(cuda, sd, weight_format=fmt, max_tokens=M)
     x = workloads.activations(M, H, seed=7391 + M, device=cuda)
@@ -313,16 +316,18 @@ def test_prefill_bitwise_deterministic(pkg, cuda, fmt, H, I, M):
 
 
 @pytest.mark.parametrize("fmt", ["bf16", "bfp8", "bf4"])
-@pytest.mark.parametrize("H,I,M", [(1024, 3072, 16), (1024, 3072, 64), (1024, 4352, 2048)])
+@pytest.mark.parametrize("H,I,M", [(1024, 3072, 16), (1024, 3072, 64), (1024, 4352, 2048), (4352, 10240, 2048)])
 def test_graph_capture_replays(pkg, cuda, fmt, H, I, M):
     """A forward captured in a HIP graph and replayed five times on new inputs, each replay
-    equal to the eager forward: the weight-streaming kernels at 16 tokens, the tiled kernels at 64
-    tokens (every tile split, padding blocks) and at 2048 tokens with split pieces (their arrival
-    counters must be back at zero after every replay)."""
+    equal to the eager forward: the weight-streaming kernels at 16 tokens (their arrival counters must
+    be back at zero after every replay), the tiled kernels at 64 tokens (every down tile split) and
+    at 2048 tokens with every down tile split and with tiles split behind whole rounds."""
     import torch
     from qwen_mlp_amd import workloads
 
     print(f"case graph {fmt} H={H} I={I} M={M}", flush=True)
+    if H == 4352:
+        assert_splits_behind_whole_rounds(pkg, fmt, H, I, M)
     sd = workloads.state_dict(H, I, layer=4, device=cuda)
     mlp = pkg.Qwen36MLP(cuda, sd, weight_format=fmt, max_tokens=M)
     static_x = workloads.activations(M, H, seed=1, device=cuda)
@@ -390,22 +395,21 @@ def test_shape_errors(pkg, cuda):
 @pytest.mark.parametrize("fmt", ["bf16", "bfp8", "bf4"])
 @pytest.mark.parametrize("H,I,M", [(1024, 3072, 2048), (5120, 17408, 256), (1024, 3072, 200), (1024, 3072, 33),
                                    (1024, 4352, 2048), (5120, 512, 2048), (6144, 2048, 2048), (5376, 2048, 2048),
+                                   (4352, 10240, 2048),
                                    (1024, 41728, 160), (1024, 3072, 2049), (2048, 2048, 4100)])
 def test_prefill_tiled(pkg, cuda, fmt, H, I, M):
     """Many-token forwards (the LDS-tiled matrix-core kernels): a full 2048-token chunk, the 27B
     shape at 256 tokens, a token count that leaves a partial token block, the narrowest width that
     takes this path (one partial block in each projection), chunks longer than 2048 tokens with a
-    ragged last block (2049: 204 gate/up tiles, fewer than one round; 4100: 264 tiles in each
-    projection, one whole round and 8 tiles in 4 pieces that meet in the workspace's fixed-size
-    split region), and, for the block-float formats,
-    shapes whose tiles do not fill whole rounds of a 256-CU GPU, so that the tiles beyond the last
-    whole round split their K range into pieces that meet in the workspace: gate/up at I = 4352
-    (16 tiles in 4 pieces) and I = 41728 (70 tiles in 3 pieces, block order left as is), down at
-    H = 5120, K = 512 and H = 6144 (2 pieces) and at H = 5376 (80 tiles in 3 pieces)."""
+    ragged last block, and shapes whose tiles do not fill whole rounds of a 256-CU GPU: H = 4352, I =
+    10240 splits the tiles beyond its whole rounds in both projections; I = 4352 and I = 41728 split
+    every down tile, I = 512 every gate/up tile; H = 6144 and H = 5376 run whole tiles only."""
     import torch
     from qwen_mlp_amd import workloads
 
     print(f"case prefill {fmt} H={H} I={I} M={M}", flush=True)
+    if H == 4352:
+        assert_splits_behind_whole_rounds(pkg, fmt, H, I, M)
     sd = workloads.state_dict(H, I, layer=8, device=cuda)
     mlp = pkg.Qwen36MLP(cuda, sd, weight_format=fmt, max_tokens=M)
     x = workloads.activations(M, H, seed=4242 + M, gain=False, device=cuda)
@@ -419,15 +423,17 @@ def test_prefill_tiled(pkg, cuda, fmt, H, I, M):
 
 
 @pytest.mark.parametrize("fmt", ["bf16", "bfp8", "bf4"])
-def test_fp32_residual_stream(pkg, cuda, fmt):
+@pytest.mark.parametrize("H,I", [(6144, 2048), (4352, 10240)])
+def test_fp32_residual_stream(pkg, cuda, fmt, H, I):
     """An fp32 residual stream (out = residual + MLP(x), the residual read as fp32) at every kind of
-    dispatch: the weight-streaming kernel (16 tokens), the 16x16 tiled kernels (200 tokens), and at
-    2048 tokens the 32x32 kernel's down projection whose last tiles split K into pieces (block-float
-    formats; bf16 weights take the 16x16 kernel there too); then in place (out = residual)."""
+    dispatch: the weight-streaming kernel (16 tokens), and the tiled kernel's down projection split
+    from the first tile on (200 tokens), whole (2048 tokens, H = 6144) and split behind whole rounds
+    (2048 tokens, H = 4352); then in place (out = residual)."""
     import torch
     from qwen_mlp_amd import workloads
 
-    H, I = 6144, 2048
+    if H == 4352:
+        assert_splits_behind_whole_rounds(pkg, fmt, H, I, 2048)
     sd = workloads.state_dict(H, I, layer=21, device=cuda)
     mlp = pkg.Qwen36MLP(cuda, sd, weight_format=fmt, max_tokens=2048)
     hw = _host_weights(pkg, sd, fmt)
@@ -449,8 +455,9 @@ def test_fp32_residual_stream(pkg, cuda, fmt):
 @pytest.mark.parametrize("fmt", ["bf16", "bfp8", "bf4"])
 def test_rmsnorm_prologue(pkg, cuda, fmt):
     """h + MLP(rmsnorm(h) * (1 + w)) against the oracle's composition (the norm output rounded to
-    bf16 as the reference's separate norm produces it), across every dispatch width: fused into
-    the M <= 32 weight-streaming kernel, a separate pass for the others; then in place (out = h)."""
+    bf16 as the reference's separate norm produces it), across every dispatch width: a pass of its own
+    before the M <= 32 weight-streaming kernel and for bf16 weights, with the fp16 conversion for
+    block-float weights above; then in place (out = h)."""
     import torch
     from qwen_mlp_amd import workloads
 

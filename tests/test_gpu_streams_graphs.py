@@ -1,8 +1,9 @@
 """Concurrent forwards on two streams and HIP-graph capture of whole layer stacks.
 
-* Two streams running many-token forwards at once: the split tiles of the matrix-core kernels
-  meet by last arrival, so no block waits for another and the two kernels' blocks may interleave
-  on the CUs in any way; every output must equal the eager, one-at-a-time result bit for bit.
+* Two streams running forwards at once: partial sums meet by last arrival (up to 32 tokens) or in
+  the next launch (the split tiles of more), so no block waits for another and the two streams'
+  blocks may interleave on the CUs in any way; every output must equal the eager, one-at-a-time
+  result bit for bit.
 * ``torch.cuda.graph(g)`` with no stream argument (torch's own capture stream), and a graph
   replayed after the shared workspace grew: the replaced workspace stays alive.
 * The 64-layer bfp8 stack (27B, 16 tokens, the decoder's RMSNorm -> MLP -> residual chain)
@@ -12,6 +13,8 @@
 """
 import pytest
 
+from parity_helpers import assert_splits_behind_whole_rounds
+
 pytestmark = pytest.mark.gpu
 
 H27, I27 = 5120, 17408
@@ -19,17 +22,20 @@ H27, I27 = 5120, 17408
 
 @pytest.mark.parametrize("fmt,H,I,M", [("bfp8", H27, I27, 16), ("bf4", H27, I27, 16), ("bfp8", H27, I27, 2048),
                                        ("bfp8", H27, I27, 64), ("bf4", 1024, 4352, 2048), ("bf16", 1024, 4352, 2048),
-                                       ("bfp8", 5376, 2048, 2048)])
+                                       ("bfp8", 5376, 2048, 2048), ("bf16", 4352, 10240, 2048),
+                                       ("bf4", 4352, 10240, 2048)])
 def test_two_streams_concurrent_forwards(pkg, cuda, fmt, H, I, M):
     """Forwards of two layers issued alternately on two streams with no synchronisation between
     them.  27B at 16 tokens: the split-K weight-streaming kernels, whose partial sums meet by last
-    arrival in per-stream counters; 27B at 2048 tokens: 64 gate/up and 64 down tiles in 4 pieces;
-    27B at 64 tokens: every tile split; I = 4352: 16 gate/up tiles in 4 pieces; H = 5376: 80 down
-    tiles in 3 pieces."""
+    arrival in per-stream counters; 27B at 2048 tokens and H = 4352, I = 10240: tiles split behind
+    whole rounds in both projections; 27B at 64 tokens: every tile split; I = 4352: every down tile
+    split; H = 5376: whole tiles."""
     import torch
     from qwen_mlp_amd import workloads
 
     print(f"case two streams {fmt} H={H} I={I} M={M}", flush=True)
+    if M == 2048 and (H, I) in ((H27, I27), (4352, 10240)):
+        assert_splits_behind_whole_rounds(pkg, fmt, H, I, M)
     pool = pkg.WorkspacePool()
     mlps = [pkg.Qwen36MLP(cuda, workloads.state_dict(H, I, layer=70 + i, device=cuda), weight_format=fmt,
                           max_tokens=M, pool=pool) for i in range(2)]
