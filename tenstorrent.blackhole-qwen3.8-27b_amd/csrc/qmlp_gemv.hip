@@ -745,7 +745,9 @@ static size_t gemv_lds_bytes(const GemvPlan& pl, int nmat, int mg) {
 // whatever the token groups (fitted on MI355X to the measured 27B-shape splits: at 16 tokens
 // gate/up 2 K splits beat 4, at 32 tokens 4 beat 3, and down 8 beat 10; charging S - 1 picks the
 // same splits there); splits using fewer than all CUs pay for it through their larger U.  K
-// splits may differ by one superblock.
+// splits may differ by one superblock.  The fit is to bfp8: a bf4 unit is half as many bytes and a
+// bf16 unit nearly twice, and the model does not know.  Some splits are level in it (gate/up of
+// 8704 x 5120 at 16 tokens: 16.56 for 4 K splits, 16.60 for 2).
 int plan_gemv(int rows, int K, int nmat, int mg, int num_cus, GemvPlan* out) {
   if (rows <= 0 || K <= 0 || rows % kTileRows || K % kSuperK || (mg != 1 && mg != 2) || (nmat != 1 && nmat != 2))
     return -1;

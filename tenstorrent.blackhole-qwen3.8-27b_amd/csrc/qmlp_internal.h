@@ -102,7 +102,7 @@ struct ForwardArgs {
   uint8_t* ws;
   int M, H, I, fmt;
   int out_f32, res_f32;  // fp32 output / fp32 residual instead of bf16
-  const void* normw;     // RMSNorm prologue: bf16 [H] weight (gain 1 + w), or null
+  const void* normw;     // the RMSNorm to apply to x first: bf16 [H] weight (gain 1 + w), or null
   float eps;
   bool normed;           // x holds rows that the RMSNorm pass wrote
 };
@@ -124,7 +124,7 @@ bool stream_supported(int M, int H, int I, int num_cus);
 int launch_forward_stream(const ForwardArgs& a, int num_cus, hipStream_t s);
 
 // Argument validation and dispatch shared by every forward entry point (qmlp_abi.hip).  `fn` names
-// the entry point in error messages; normw != null selects the RMSNorm prologue.
+// the entry point in error messages; normw != null selects the RMSNorm.
 int forward_impl(const char* fn, const void* x, const void* wg, const void* wu, const void* wd, const void* residual,
                  void* out, void* ws, size_t ws_bytes, int M, int H, int I, int fmt, int flags, const void* normw,
                  float eps, hipStream_t stream);

@@ -282,8 +282,12 @@ __global__ __launch_bounds__(512) void tiled32_kernel(TlParams p) {
   const uint32_t lp0 = (uint32_t)(32 * hk + (lane & 15)), lp1 = lp0 + 16u;
   const uint32_t wv = (uint32_t)((lane >> 4) & 1) * (uint32_t)tile_bytes;  // the lane's tile
   // Weights that several token blocks read stay in L2 for them; with one token block (ONCE) they are
-  // read once and pass it by (27B layer at 64 tokens: bf16 127.4 -> 121.8 us, bfp8 82.4 -> 81.4; with
-  // several token blocks 1-6 % slower).
+  // read once and pass it by.  27B, eight layers in turn, us per layer without -> with: bf16 127.2 ->
+  // 120.4 at 64 tokens and 139.2 -> 131.3 at 96; bfp8 79.8 -> 78.2 at 33, 83.1 -> 82.1 at 64 and 104.8 ->
+  // 104.4 at 96 (its down launch alone is 0.6 us slower, the layer faster); bf4, whose down launch only
+  // uses it, level: 76.0 / 76.2, 79.8 / 80.5 and 95.6 / 94.9.  Two or three layers in turn, which the
+  // memory-side cache holds in part, differ by up to 6 us either way.  With several token blocks
+  // 1-6 % slower.
   constexpr int POL = ONCE ? 2 : 0;  // buffer cache policy: non-temporal
   auto wload = [&](Tl32Stage<WF, NM>& st, int step) {
     const int sc = kb + min(step, nst - 1);
@@ -771,7 +775,9 @@ static int launch_tiled32(TlParams p, const TilePlan& t, hipStream_t s) {
 }
 
 // Weights one token block reads pass the L2 by only where a load takes whole 16-byte pieces: bf4's
-// 8-byte loads of two steps share their lines (64 tokens: 85.9 against 80.7 us).
+// 8-byte loads of two steps share their lines (64 tokens: 85.9 against 80.7 us).  Taller tiles are the
+// one token block of few plans (27B: down at 129-160 tokens) and gain less there: bf16 layer 156.5 ->
+// 155.4 us, bfp8 134.7 -> 134.1, bf4 level.
 template <int WF, int MODE, int MG>
 static int launch_height(const TlParams& p, const TilePlan& t, hipStream_t s) {
   if constexpr (WF != 2 && MG <= 3)
