@@ -620,7 +620,7 @@ __global__ __launch_bounds__(256) void sum_kernel(TlParams p, int mg) {
 // 2048 at the 27B shapes (H = 5120, I = 17408), every tile height and the splits within 1.4 x the
 // best estimate, about 500 points per mode and format, fitted to 3-5 % rms with the points near the
 // fastest weighted most.  The plans chosen are 0.7 % slower on average than the fastest measured there
-// (0.9-2.1 % in a later run on another box, at most 12 %, below 100 tokens).  At other shapes
+// (0.9-2.1 % in a later run on another card, at most 12 %, below 100 tokens).  At other shapes
 // (H = 1024-5120, I = 3072-16640, 48-2048 tokens) the estimates are up to a fifth too high, as tiles
 // over a short K overlap their ends, and the plans are 0.3 (bf4), 1.0 (bf16) and 1.3 % (bfp8) slower
 // than the fastest for gate/up, 1.2-1.7 and 3.5 % (bf16) for down, single ones by up to 24 %.
